@@ -155,7 +155,7 @@ Layout layout(const Dims& d) {
   const bool sp = d.sparse;
   L.base = take(sp ? (size_t)d.N * d.C * d.s : 0);
   L.ag = take(sp ? nk * d.C * d.so : 0);
-  L.ortho = take((size_t)(d.E * (d.E - 1) / 2 + 1) * sizeof(float));
+  L.ortho = take((size_t)ortho_tiles(d.E, d.r) * sizeof(float));
   // split-K partials of the key product (with or without adapter columns)
   // and of the value product (K = F, or F + Kx in FUSED mode); one region
   // serves both, as they run one after the other

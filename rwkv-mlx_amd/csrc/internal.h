@@ -334,6 +334,8 @@ hipError_t launch_lora_grouped(int dtype, const void* x, const void* at, const v
 hipError_t launch_combine(int dtype, const void* base, const void* ag, const int* inds, const void* gates,
                           const int* inv, const void* resid, void* out, int N, int C, int k, hipStream_t s,
                           bool mixed = false);
+// `part`: ortho_tiles(E, r) floats of scratch.
+int ortho_tiles(int E, int r);
 hipError_t launch_ortho(int dtype, const void* A, int E, int C, int r, float* part, float* out, hipStream_t s);
 // y = fp32(x) for n (a multiple of 8) elements of a 16-bit dtype
 hipError_t launch_widen(int dtype, const void* x, float* y, size_t n, hipStream_t s);
