@@ -161,8 +161,10 @@ Layout layout(const Dims& d) {
   // serves both, as they run one after the other
   const bool fused = !d.sparse;
   size_t sk = gemm_partial_bytes(d.dtype, d.N, d.F, d.F, d.C, false);
-  if (fused && !router_fuses_adapters(d.N, d.C, d.E, d.r, d.dtype))
+  if (fused && !router_fuses_adapters(d.N, d.C, d.E, d.r, d.dtype)) {
     sk = std::max(sk, gemm_partial_bytes(d.dtype, d.N, d.F + d.kx, d.F, d.C, true));
+    sk = std::max(sk, gemm_partial_bytes(d.dtype, d.N, d.kx, 0, d.C, true));  // the adapter columns alone
+  }
   sk = std::max(sk, gemm_partial_bytes(d.dtype, d.N, d.C, d.C, d.F + (fused ? d.kx : 0), false));
   sk = std::max(sk, gemm_partial_bytes(d.dtype, d.N, d.C, d.C, d.F, false));
   L.splitk = take(sk);

@@ -12,13 +12,17 @@
 // token by the router pass or by shift_mix_kernel, not per output tile.
 // relu² and the residual add run in the epilogue.
 //
-// Kernel structure (256 threads = 4 waves in a 2x2 grid, BM x BN tile):
-//   * K is walked in 128-byte slices (64 fp16/bf16 or 32 fp32 elements) that
-//     buffer_load_dwordx4 ... lds writes straight into an S-deep LDS ring.  LDS
-//     rows are 128 bytes, unpadded, with the 16-byte chunk index XOR-swizzled
-//     by row so the MFMA fragment reads are free of bank conflicts.
-//   * Each wave computes (BM/2) x (BN/2) with v_mfma_f32_32x32x16_{f16,bf16}
-//     (v_mfma_f32_32x32x2f32 for fp32).
+// 16-bit products run the pipelined tiles of gemm_pipe.h (planned here,
+// plan_pipe); this file's kernel keeps fp32 products, the fp16 layer with fp32
+// adapters (MX) and 16-bit products of at most 64 rows.
+//
+// Kernel structure (BM x BN tile, WGM x WGN waves and LW load-only waves):
+//   * K is walked in slices of RB bytes per row that buffer_load_dwordx4 ... lds
+//     writes straight into an S-deep LDS ring.  LDS rows are unpadded, with the
+//     16-byte chunk index XOR-swizzled by row so the MFMA fragment reads are
+//     free of bank conflicts.
+//   * Each wave computes its part of the tile with v_mfma_f32_32x32x16_{f16,bf16}
+//     or 16x16x32 (v_mfma_f32_32x32x2f32 for fp32).
 //   * The epilogue converts the tile into its own LDS buffer, then writes it
 //     out with 16-byte coalesced stores while the next tile's slices load.
 //   * Workgroups are persistent (one per CU); each XCD owns a contiguous run
@@ -27,6 +31,7 @@
 //     L2.
 #include <stdlib.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -798,6 +803,63 @@ TilePlan plan_tiles(int elem, int epi, int m, int n, int n_key, int k_total) {
   return pl;
 }
 
+// ---- 16-bit products: the tile of gemm_pipe.h ----
+// Microseconds of one 64-wide K slice of a tile: `slice` per tile with every CU
+// busy (tiles of which two share a CU: the pair's time over two), `alone` where
+// a CU holds one tile, both measured at K = 8192 with 256 to 4096 tiles (bf16,
+// 16384 x 2048 and 200 to 2031 rows).
+struct PipeTile {
+  int bm, bn, per_cu;
+  double slice, alone;
+};
+constexpr PipeTile kPipeTiles[] = {
+    {256, 256, 1, 1.57, 1.57}, {256, 192, 1, 1.25, 1.25}, {256, 128, 1, 0.87, 0.87}, {128, 192, 1, 0.72, 0.72},
+    {128, 128, 1, 0.53, 0.53}, {128, 128, 2, 0.52, 0.60}, {128, 64, 2, 0.35, 0.30},  {64, 64, 2, 0.22, 0.21},
+};
+
+struct PipePlan {
+  int cfg;    // of kPipeTiles, -1: none fits
+  int ks;     // K splits
+  double us;  // the model's time
+};
+
+// The tile (and K split) with the least modelled time: rounds of tiles over
+// the CUs times a tile's slices, plus 1 us a round for its epilogue.  With
+// fewer tiles than CUs a slice takes down to 0.7 of its time (L2 and the
+// infinity cache serve fewer CUs).  A split adds the reduction's launch and the
+// fp32 partials' traffic.  A tile never straddles the key / adapter column
+// boundary.  groups: row groups (each may end in a partial tile) or K groups;
+// ld: the operands' row length where it can be long (a tile's rows are
+// addressed with 32 bits).
+PipePlan plan_pipe(int mode, int m, int n, int n_key, int nkt, int groups = 1, long long ld = 0) {
+  const int cus = num_cus();
+  PipePlan best{-1, 1, 0.};
+  for (int c = 0; c < (int)(sizeof(kPipeTiles) / sizeof(kPipeTiles[0])); ++c) {
+    const PipeTile& t = kPipeTiles[c];
+    if (n % t.bn || n_key % t.bn || ld * std::max(t.bm, t.bn) * 2 > 0xFFFFFFF0ll) continue;
+    long long tiles = (long long)((m + t.bm - 1) / t.bm) * (n / t.bn);
+    if (mode == PIPE_GRP) tiles += (long long)(groups / 2) * (n / t.bn);
+    if (mode == PIPE_GK) tiles *= groups;
+    const bool split = mode == PIPE_DENSE && (c == 4 || c == 6 || c == 7);
+    for (int ks = 1; ks <= (split ? 16 : 1) && (ks == 1 || nkt / ks >= 4); ++ks) {
+      const long long items = tiles * ks;
+      if (ks > 1 && items > (long long)cus * t.per_cu) break;
+      const long long slots = (long long)cus * t.per_cu, rest = items % slots;
+      const double nk = (double)((nkt + ks - 1) / ks);
+      const double fill = items >= cus ? 1.0 : 0.7 + 0.3 * (double)items / cus;
+      double us = (double)(items / slots) * t.per_cu * (nk * t.slice + 1.0);
+      if (rest > cus) us += t.per_cu * (nk * t.slice + 1.0);
+      else if (rest > 0) us += nk * t.alone * fill + 1.0;
+      if (ks > 1) us += 4.0 + (double)ks * m * n * 8.0 / 3.5e6;
+      if (best.cfg < 0 || us < best.us) best = PipePlan{c, ks, us};
+    }
+  }
+  return best;
+}
+
+// Whether a 16-bit product runs this file's 64-row tiles (codes 8 and 9).
+bool small_rows_plan(const TilePlan& pl) { return pl.t == 8 || pl.t == 9; }
+
 // With `deferred`, a split product leaves its partials in p.part for the
 // caller to reduce (in ascending split order) and reports the split count.
 // LW: waves that only issue loads (more loads in flight per CU).
@@ -822,9 +884,26 @@ hipError_t dispatch_tile(const GemmParams<T>& p, hipStream_t s, const TilePlan* 
   const TilePlan pl = given ? *given : plan_tiles((int)sizeof(T), EPI, p.m, p.n, p.n_key, p.k1 + (EXT ? p.k2 : 0));
   const int t = pl.t;
   if (deferred) *deferred = 1;
-  if (vs_enabled() && (t == 3 || t == 5 || t == 6)) {
-    const hipError_t e = gemm_vs_run<T>(p, t, EPI, EXT, MX, s);
-    if (e != hipErrorNotSupported) return e;
+  if constexpr (MX) {
+    if (vs_enabled() && t == 6) {
+      const hipError_t e = gemm_vs_run<T>(p, t, EPI, EXT, MX, s);
+      if (e != hipErrorNotSupported) return e;
+    }
+  } else if constexpr (sizeof(T) == 2) {
+    if (t == 9 && fits(16)) return run_small<T, 64, 16, EPI, EXT, 0, 4, 1, 16>(p, pl.ks, s, deferred);
+    if (t == 8 && fits(16)) {
+      if (p.k1 % 128 == 0 && (!EXT || p.k2 % 128 == 0)) return run<T, 64, 16, 4, 1, 3, EPI, EXT, 16, 0, 256>(p, s, false);
+      return run<T, 64, 16, 4, 1, 3, EPI, EXT, 16, 0, 128>(p, s, false);
+    }
+    const PipePlan pp = plan_pipe(PIPE_DENSE, p.m, p.n, EPI == EPI_KEYAD ? p.n_key : p.n, (p.k1 + (EXT ? p.k2 : 0)) / 64);
+    if (pp.cfg < 0) return hipErrorInvalidValue;
+    GemmParams<T> q = p;
+    q.ksplit = pp.ks;
+    if (EPI != EPI_RESID) q.resid = nullptr;
+    const hipError_t e = pipe_run<T>(q, pp.cfg, EPI == EPI_KEY || EPI == EPI_KEYAD ? EPI_KEYAD : EPI_STORE, PIPE_DENSE, s);
+    if (e != hipSuccess || pp.ks <= 1) return e;
+    launch_kernel((splitk_reduce_kernel<T, EPI>), dim3((p.m * (p.n / 4) + 255) / 256), dim3(256), 0, s, q);
+    return hipGetLastError();
   }
   if constexpr (MX) {
     // fp32 out tiles: the 256-row tiles' fp32 output does not fit LDS beside
@@ -842,48 +921,17 @@ hipError_t dispatch_tile(const GemmParams<T>& p, hipStream_t s, const TilePlan* 
     }
     return hipErrorInvalidValue;
   }
-  if constexpr (sizeof(T) == 2)
-    if (t == 9 && fits(16)) return run_small<T, 64, 16, EPI, EXT, 0, 4, 1, 16>(p, pl.ks, s, deferred);
-  if (t == 7) {
-    if (!fits(pl.bn)) return hipErrorInvalidValue;
-    // plain products with long work items (8+ K slices each: the backward's
-    // token-contracted products) are load-bound: 4 more waves issue loads
-    if constexpr (EPI == EPI_STORE && !EXT) {
-      const int items_k = p.k1 / (128 / (int)sizeof(T)) / (pl.ks > 1 ? pl.ks : 1);
-      if (items_k >= 8) {
-        if constexpr (sizeof(T) == 2)
-          if (pl.bn == 128) return run_small<T, 64, 128, EPI, EXT, 4>(p, pl.ks, s, deferred);
-        return run_small<T, 64, 64, EPI, EXT, 4>(p, pl.ks, s, deferred);
+  if constexpr (sizeof(T) == 4) {
+    if (t == 7) {
+      if (!fits(pl.bn)) return hipErrorInvalidValue;
+      // plain products with long work items (8+ K slices each: the backward's
+      // token-contracted products) are load-bound: 4 more waves issue loads
+      if constexpr (EPI == EPI_STORE && !EXT) {
+        const int items_k = p.k1 / (128 / (int)sizeof(T)) / (pl.ks > 1 ? pl.ks : 1);
+        if (items_k >= 8) return run_small<T, 64, 64, EPI, EXT, 4>(p, pl.ks, s, deferred);
       }
+      return run_small<T, 64, 64, EPI, EXT>(p, pl.ks, s, deferred);
     }
-    if constexpr (sizeof(T) == 2)
-      if (pl.bn == 128) return run_small<T, 64, 128, EPI, EXT>(p, pl.ks, s, deferred);
-    return run_small<T, 64, 64, EPI, EXT>(p, pl.ks, s, deferred);
-  }
-  if constexpr (sizeof(T) == 2) {
-    if (t == 8 && fits(16)) {
-      if (p.k1 % 128 == 0 && (!EXT || p.k2 % 128 == 0)) return run<T, 64, 16, 4, 1, 3, EPI, EXT, 16, 0, 256>(p, s, false);
-      return run<T, 64, 16, 4, 1, 3, EPI, EXT, 16, 0, 128>(p, s, false);
-    }
-    // the relu² products in 64-element slices, two 64 KB stages (the skewed
-    // layer's key product 80.0 against 83.2 us, D=2048's 520 against 525;
-    // the value products measured slower so: 510 against 485 us at D=2048)
-    if constexpr (EPI == EPI_KEY)
-      if (t == 10 && fits(256) && p.k1 % 64 == 0 && (!EXT || p.k2 % 64 == 0))
-        return run<T, 256, 256, 2, 4, 2, EPI, EXT, 32, 0, 128>(p, s, false);
-    if (t == 10 && fits(256) && p.k1 % 32 == 0 && (!EXT || p.k2 % 32 == 0))
-      return run<T, 256, 256, 2, 4, 5, EPI, EXT, 32, 0, 64>(p, s, false);
-    if constexpr (EPI != EPI_KEYAD)
-      if (t == 3 && fits(192)) return run<T, 256, 192, 4, 2, 2, EPI, EXT>(p, s, false);
-    if ((t == 5 || t == 10) && fits(128)) return run<T, 256, 128, 4, 2, 2, EPI, EXT>(p, s, false);
-    if (t == 6 && fits(96)) {
-      if (p.k1 % 128 == 0 && (!EXT || p.k2 % 128 == 0)) return run<T, 128, 96, 2, 2, 2, EPI, EXT, 16, 10, 256>(p, s, false);
-      return run<T, 128, 96, 2, 2, 4, EPI, EXT, 16, 3>(p, s, true);
-    }
-    if (t == 1 && fits(128)) return run<T, 128, 128, 2, 2, 4, EPI, EXT>(p, s, true);
-    if (!fits(64)) return hipErrorInvalidValue;
-    return run<T, 128, 64, 2, 2, 4, EPI, EXT>(p, s, true);
-  } else {
     if (t == 1 && fits(128)) return run<T, 128, 128, 2, 2, 3, EPI, EXT>(p, s, true);
     if (!fits(64)) return hipErrorInvalidValue;
     return run<T, 128, 64, 2, 2, 4, EPI, EXT>(p, s, true);
@@ -916,6 +964,10 @@ bool value_plan_mixed_ok(int m, int n, int k_total) {
 
 size_t gemm_partial_bytes(int dtype, int m, int n, int n_key, int k_total, bool keyad) {
   const TilePlan pl = plan_tiles(dtype == 0 ? 4 : 2, keyad ? EPI_KEYAD : EPI_KEY, m, n, n_key, k_total);
+  if (dtype != 0 && !small_rows_plan(pl)) {
+    const PipePlan pp = plan_pipe(PIPE_DENSE, m, n, keyad ? n_key : n, k_total / 64);
+    return pp.ks > 1 ? (size_t)pp.ks * m * n * sizeof(float) : 0;
+  }
   return (pl.t == 7 || pl.t == 9) && pl.ks > 1 ? (size_t)pl.ks * m * n * sizeof(float) : 0;
 }
 
@@ -933,35 +985,14 @@ hipError_t launch_shift_mix(int dtype, const void* x, const void* xprev, const v
 
 // Whether the key product with adapter columns runs as two launches, the key
 // columns alone and then the adapter columns alone (n_key = 0).  One launch
-// rounds the combined tile count up to whole rounds of tiles over the CUs:
-// at D=2048 (F = 8192, Kx = 512, 16384 tokens) 2176 tiles of 256x256 on 256
-// CUs run as 9 rounds where the key columns alone fill 8 exactly.  Two
+// rounds the combined tile count up to whole rounds of tiles over the CUs; two
 // launches round each product up on its own tiles (the adapter product takes
-// smaller ones).  Tile area per round stands for time; only wide key
-// products (256x256 tiles) are considered.
+// smaller ones) and cost another launch, about 4 us.
 bool split_key_adapters(int elem, int N, int C, int F, int kx) {
-  auto dims = [](int t, int& bm, int& bn) {
-    switch (t) {
-      case 10: bm = 256; bn = 256; return true;
-      case 3: bm = 256; bn = 192; return true;
-      case 5: bm = 256; bn = 128; return true;
-      case 6: bm = 128; bn = 96; return true;
-      case 1: bm = 128; bn = 128; return true;
-      case 2: bm = 128; bn = 64; return true;
-      default: return false;  // split-K and decode tiles
-    }
-  };
-  const TilePlan k = plan_tiles(elem, EPI_KEY, N, F, F, C);
-  const TilePlan c = plan_tiles(elem, EPI_KEYAD, N, F + kx, F, C);
-  const TilePlan a = plan_tiles(elem, EPI_KEYAD, N, kx, 0, C);
-  int bmk, bnk, bmc, bnc, bma, bna;
-  if (k.t != 10 || !dims(k.t, bmk, bnk) || !dims(c.t, bmc, bnc) || !dims(a.t, bma, bna)) return false;
-  const long long cus = num_cus();
-  auto cost = [&](int bm, int bn, int n) {
-    const long long tiles = (long long)((N + bm - 1) / bm) * (n / bn);
-    return (tiles + cus - 1) / cus * bm * bn;
-  };
-  return cost(bmk, bnk, F) + cost(bma, bna, kx) < cost(bmc, bnc, F + kx);
+  if (elem != 2 || small_rows_plan(plan_tiles(elem, EPI_KEYAD, N, F + kx, F, C))) return false;
+  const PipePlan k = plan_pipe(PIPE_DENSE, N, F, F, C / 64), a = plan_pipe(PIPE_DENSE, N, kx, 0, C / 64),
+                 c = plan_pipe(PIPE_DENSE, N, F + kx, F, C / 64);
+  return k.us + a.us + 4.0 < c.us;
 }
 
 hipError_t launch_cmix_key(int dtype, const void* xk, const void* wk, void* h, int N, int C, int F, const void* x,
@@ -1076,45 +1107,25 @@ hipError_t launch_cmix_value_sparse(int dtype, const void* h, const void* wv, in
   return mark(e, "cmix_value_sparse", s);
 }
 
-// Grouped product: one tile per workgroup, no split K or persistent grid.
-// The tile minimises waves x operand rows per tile (ceil(tiles / CUs) x
-// (BM + BN)): these products are bound by each CU's operand loads, and a
-// partial last wave costs as much as a full one.  Ties go to the larger
-// tile.  Candidates (16-bit): 256x192, 256x128, 128x96 (K % 128 == 0),
-// 128x128, 64x128, 64x64; fp32: 128x128, 64x64.
+// Grouped product.  16-bit: the pipelined tiles; fp32: one tile per workgroup,
+// 128x128 or 64x64 by waves x operand rows per tile (ceil(tiles / CUs) x (BM +
+// BN): these products are bound by each CU's operand loads, and a partial
+// last wave costs as much as a full one), ties to the larger.
 template <typename T, int EPI>
 hipError_t dispatch_grouped(const GemmParams<T>& p, hipStream_t s) {
-  auto fits = [&](int bn) { return p.n % bn == 0; };
-  auto tiles = [&](int bm, int bn) { return ((p.m + bm - 1) / bm + p.grp_n) * (p.n / bn); };
-  const int cus = num_cus();
-  struct Cand { int bm, bn; bool ok; };
-  const bool h = sizeof(T) == 2;
-  const Cand cands[] = {{256, 192, h && fits(192)}, {256, 128, h && fits(128)},
-                        {128, 96, h && fits(96) && p.k1 % 128 == 0}, {128, 128, fits(128)},
-                        {64, 128, h && fits(128)}, {64, 64, fits(64)}};
-  int best = -1;
-  long long best_cost = 0;
-  for (int i = 0; i < (int)(sizeof(cands) / sizeof(cands[0])); ++i) {
-    if (!cands[i].ok) continue;
-    const long long waves = (tiles(cands[i].bm, cands[i].bn) + cus - 1) / cus;
-    const long long cost = waves * (cands[i].bm + cands[i].bn);
-    if (best < 0 || cost < best_cost) {
-      best = i;
-      best_cost = cost;
-    }
-  }
-  if (best < 0) return hipErrorInvalidValue;
   if constexpr (sizeof(T) == 2) {
-    switch (best) {
-      case 0: return run<T, 256, 192, 4, 2, 2, EPI, false, 32, 0, 128, false, false, true>(p, s, false);
-      case 1: return run<T, 256, 128, 4, 2, 2, EPI, false, 32, 0, 128, false, false, true>(p, s, false);
-      case 2: return run<T, 128, 96, 2, 2, 2, EPI, false, 16, 10, 256, false, false, true>(p, s, false);
-      case 3: return run<T, 128, 128, 2, 2, 4, EPI, false, 32, 0, 128, false, false, true>(p, s, false);
-      case 4: return run<T, 64, 128, 2, 2, 3, EPI, false, 32, 0, 128, false, false, true>(p, s, false);
-      default: return run<T, 64, 64, 2, 2, 3, EPI, false, 32, 0, 128, false, false, true>(p, s, false);
-    }
+    const PipePlan pp = plan_pipe(PIPE_GRP, p.m, p.n, p.n, p.k1 / 64, p.grp_n);
+    if (pp.cfg < 0) return hipErrorInvalidValue;
+    return pipe_run<T>(p, pp.cfg, EPI == EPI_KEY ? EPI_KEYAD : EPI_STORE, PIPE_GRP, s);
   } else {
-    if (best == 3) return run<T, 128, 128, 2, 2, 3, EPI, false, 32, 0, 128, false, false, true>(p, s, false);
+    const int cus = num_cus();
+    auto cost = [&](int bm, int bn) -> long long {
+      const int tiles = ((p.m + bm - 1) / bm + p.grp_n) * (p.n / bn);
+      return (long long)((tiles + cus - 1) / cus) * (bm + bn);
+    };
+    if (p.n % 128 == 0 && cost(128, 128) <= cost(64, 64))
+      return run<T, 128, 128, 2, 2, 3, EPI, false, 32, 0, 128, false, false, true>(p, s, false);
+    if (p.n % 64) return hipErrorInvalidValue;
     return run<T, 64, 64, 2, 2, 3, EPI, false, 32, 0, 128, false, false, true>(p, s, false);
   }
 }
@@ -1170,11 +1181,13 @@ hipError_t launch_gemm_grouped_k(int dtype, const void* a, int lda, const void* 
     p.m = m; p.n = n; p.out = (T*)out; p.ldo = ldo; p.n_key = n;
     p.gk_off = koff; p.gk_n = n_groups; p.gk_ostride = ostride;
     hipError_t e;
-    if (n % 128 == 0) {
-      if constexpr (sizeof(T) == 2)
-        e = run<T, 128, 128, 2, 2, 4, EPI_STORE, false, 32, 0, 128, false, false, false, false, true>(p, s, false);
-      else
-        e = run<T, 128, 128, 2, 2, 3, EPI_STORE, false, 32, 0, 128, false, false, false, false, true>(p, s, false);
+    if constexpr (sizeof(T) == 2) {
+      // (an output's K range is read on the device: planned at the average)
+      const PipePlan pp = plan_pipe(PIPE_GK, m, n, n, std::max(1, lda / n_groups / 64), n_groups,
+                                    std::max(lda, ldb));
+      e = pp.cfg < 0 ? hipErrorInvalidValue : pipe_run<T>(p, pp.cfg, EPI_STORE, PIPE_GK, s);
+    } else if (n % 128 == 0) {
+      e = run<T, 128, 128, 2, 2, 3, EPI_STORE, false, 32, 0, 128, false, false, false, false, true>(p, s, false);
     } else {
       e = run<T, 64, 64, 2, 2, 3, EPI_STORE, false, 32, 0, 128, false, false, false, false, true>(p, s, false);
     }
@@ -1185,6 +1198,10 @@ hipError_t launch_gemm_grouped_k(int dtype, const void* a, int lda, const void* 
 
 size_t gemm_nt_partial_bytes(int dtype, int m, int n, int k_total, int hint) {
   const TilePlan pl = gemm_nt_plan(dtype, m, n, k_total, hint);
+  if (dtype != 0 && !small_rows_plan(pl)) {
+    const PipePlan pp = plan_pipe(PIPE_DENSE, m, n, n, k_total / 64);
+    return pp.ks > 1 ? (size_t)pp.ks * m * n * sizeof(float) : 0;
+  }
   return (pl.t == 7 || pl.t == 9) && pl.ks > 1 ? (size_t)pl.ks * m * n * sizeof(float) : 0;
 }
 

@@ -275,4 +275,12 @@ constexpr bool out_in_ring() {
 template <typename T>
 hipError_t gemm_vs_run(const GemmParams<T>& p, int tile, int epi, bool ext, bool mx, hipStream_t s);
 
+// The pipelined 16-bit tiles (gemm_pipe.h): tile `cfg` of kPipeTiles with the
+// epilogue EPI_STORE (+ the residual where p.resid is set) or EPI_KEYAD (relu²
+// on columns below n_key, the gate mask on the rest); p.k2 > 0: a second K
+// segment; p.ksplit > 1: fp32 partials into p.part.
+enum { PIPE_DENSE = 0, PIPE_GRP = 1, PIPE_GK = 2 };
+template <typename T>
+hipError_t pipe_run(const GemmParams<T>& p, int cfg, int epi, int mode, hipStream_t s);
+
 }  // namespace rwkvmoe

@@ -507,58 +507,29 @@ hipError_t run_vs(const GemmParams<T>& p, hipStream_t s) {
 
 }  // namespace
 
-// 256x128: 8 MFMA waves (4x2, 32x32 blocks), 8 load waves, 128-byte slices,
-// two slices in flight per load lane.
-template <typename T>
-hipError_t run_vs_256x128(const GemmParams<T>& p, int epi, bool ext, hipStream_t s) {
-  if (ext) {
-    if (epi == EPI_RESID) return run_vs<T, 256, 128, 4, 2, 32, 8, 128, 2, EPI_RESID, true, false>(p, s);
-    if (epi == EPI_STORE) return run_vs<T, 256, 128, 4, 2, 32, 8, 128, 2, EPI_STORE, true, false>(p, s);
-    return hipErrorNotSupported;
-  }
-  if (epi == EPI_RESID) return run_vs<T, 256, 128, 4, 2, 32, 8, 128, 2, EPI_RESID, false, false>(p, s);
-  if (epi == EPI_STORE) return run_vs<T, 256, 128, 4, 2, 32, 8, 128, 2, EPI_STORE, false, false>(p, s);
-  if (epi == EPI_COMBINE) return run_vs<T, 256, 128, 4, 2, 32, 8, 128, 2, EPI_COMBINE, false, false>(p, s);
-  if (epi == EPI_KEY) return run_vs<T, 256, 128, 4, 2, 32, 8, 128, 2, EPI_KEY, false, false>(p, s);
-  if (epi == EPI_KEYAD) return run_vs<T, 256, 128, 4, 2, 32, 8, 128, 2, EPI_KEYAD, false, false>(p, s);
-  return hipErrorNotSupported;
-}
-
 // Variant of a tile code (gemm.hip's numbering) in the VGPR-staged form;
 // hipErrorNotSupported when there is none (the caller keeps the ring form).
-//   6: 128x96, 4 MFMA waves (2x2, 16x16 blocks), 12 load waves, 256-byte slices
-//      (the value product: 26.9 against 30.9 us in the ring form at 4096 x 768
-//      x 3072; the 256x192 key tile measured slower in this form, 30.6
-//      against 29.3 us, and keeps the ring).  Two slices in flight per load
-//      lane: with the adapter K-extension at 4096 x 768 x 3200, 28.7-29.4 us
-//      against 30.0-30.3 us with three, 30.6-31.1 with four and 30.6-31.5
-//      with five; 8 load waves or 8 MFMA waves measured slower (30.9-37.4);
-//      the fp32-adapter product too (30.5 against 31.2-32.0 us with three)
-//   5: 256x128, 8 MFMA waves, 8 load waves (run_vs_256x128; against the ring
-//      form: 615 / 554 against 732 / 706 us for the plain key / value products
-//      at 16384 x 8192 x 2048 and 16384 x 2048 x 8192 bf16, 99 / 78 against
-//      108 / 85 us at 8192 x 4096 x 1024 and 8192 x 1024 x 4096 fp16)
+//   6: 128x96, 4 MFMA waves (2x2, 16x16 blocks), 12 load waves, 256-byte
+//      slices, two in flight per load lane (three and more measured slower):
+//      the SPARSE layer's value products (rank slices, fused combine) and the
+//      fp32-adapter product
+//   5: 256x128, 8 MFMA waves (4x2, 32x32 blocks), 8 load waves, 128-byte
+//      slices: the fused combine of wider layers
 template <typename T>
 hipError_t gemm_vs_run(const GemmParams<T>& p, int tile, int epi, bool ext, bool mx, hipStream_t s) {
   if constexpr (sizeof(T) != 2) {
     return hipErrorNotSupported;
   } else {
-    if (tile == 5 && !mx && p.k1 % 64 == 0 && (!ext || p.k2 % 64 == 0)) return run_vs_256x128<T>(p, epi, ext, s);
+    if (tile == 5 && !mx && !ext && epi == EPI_COMBINE && p.k1 % 64 == 0)
+      return run_vs<T, 256, 128, 4, 2, 32, 8, 128, 2, EPI_COMBINE, false, false>(p, s);
     if (tile == 6 && (p.k1 % 128 == 0) && (!ext || p.k2 % 128 == 0)) {
       if (mx) {
         if (epi == EPI_RESID) return run_vs<T, 128, 96, 2, 2, 16, 12, 256, 2, EPI_RESID, true, true>(p, s);
         if (epi == EPI_STORE) return run_vs<T, 128, 96, 2, 2, 16, 12, 256, 2, EPI_STORE, true, true>(p, s);
         return hipErrorNotSupported;
       }
-      if (ext) {
-        if (epi == EPI_SPARSE) return run_vs<T, 128, 96, 2, 2, 16, 12, 256, 2, EPI_SPARSE, true, false>(p, s);
-        if (epi == EPI_RESID) return run_vs<T, 128, 96, 2, 2, 16, 12, 256, 2, EPI_RESID, true, false>(p, s);
-        if (epi == EPI_STORE) return run_vs<T, 128, 96, 2, 2, 16, 12, 256, 2, EPI_STORE, true, false>(p, s);
-        return hipErrorNotSupported;
-      }
-      if (epi == EPI_RESID) return run_vs<T, 128, 96, 2, 2, 16, 12, 256, 2, EPI_RESID, false, false>(p, s);
-      if (epi == EPI_STORE) return run_vs<T, 128, 96, 2, 2, 16, 12, 256, 2, EPI_STORE, false, false>(p, s);
-      if (epi == EPI_COMBINE) return run_vs<T, 128, 96, 2, 2, 16, 12, 256, 2, EPI_COMBINE, false, false>(p, s);
+      if (ext && epi == EPI_SPARSE) return run_vs<T, 128, 96, 2, 2, 16, 12, 256, 2, EPI_SPARSE, true, false>(p, s);
+      if (!ext && epi == EPI_COMBINE) return run_vs<T, 128, 96, 2, 2, 16, 12, 256, 2, EPI_COMBINE, false, false>(p, s);
     }
     return hipErrorNotSupported;
   }

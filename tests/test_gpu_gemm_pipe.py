@@ -1,0 +1,111 @@
+"""The pipelined 16-bit products (key with relu², value) at the sizes where
+their tiles, rings and tile choice can go wrong: one K slice per tile (fewer
+than the ring holds) with many tiles per workgroup, ragged last rows, the
+smallest widths, K splits, every tile shape, the K-extension with the residual,
+and row groups that are empty, ragged or hold almost every token."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# out and h are rounded once (h twice: the product and its square), after an
+# fp32 sum whose own error is far below that
+UNIT = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}
+
+SHAPES = [(65, 64, 64), (66, 128, 64), (129, 64, 192), (200, 2048, 1024), (200, 512, 8192), (257, 192, 384),
+          (300, 320, 576), (1000, 64, 960), (2031, 1024, 3584), (4096, 768, 3072), (4100, 768, 256),
+          (8192, 1024, 4096), (9001, 256, 512), (33000, 64, 128), (70000, 64, 64)]
+
+
+@pytest.mark.parametrize("N,C,F", SHAPES)
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_key_and_value_products(device, dtype, N, C, F):
+    import torch
+    from rwkv_mlx_amd import _lib
+    dt = {"f16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    g = torch.Generator(device=device).manual_seed(N + C + F)
+    rand = lambda *s, sc=1.0: (torch.randn(*s, generator=g, device=device) * sc).to(dt)
+    x, xk = rand(1, N, C), torch.zeros(C, device=device, dtype=dt)  # x_k = 0: no token shift
+    wk, wv = rand(F, C, sc=C ** -0.5), rand(C, F, sc=F ** -0.5)
+    desc = _lib.make_desc(1, N, C, F, 1, 1, 1, dtype)
+    nb = _lib.workspace_bytes(desc)
+    ws = torch.full((nb,), 0xFF, dtype=torch.uint8, device=device)
+    h = torch.full((N + 1, F), float("nan"), dtype=dt, device=device)  # (the last row: past the end)
+    out = torch.full((N + 1, C), float("nan"), dtype=dt, device=device)
+    s = _lib.current_stream(device)
+    _lib.call("rwkvmoe_cmix_key", desc, _lib.make_tensors(x=x, x_k=xk, w_key=wk, hidden=h), ws, nb, s)
+    _lib.call("rwkvmoe_cmix_value", desc, _lib.make_tensors(hidden=h, w_value=wv, base_out=out), ws, nb, s)
+    torch.cuda.synchronize()
+    ref_h = torch.relu(x[0].double() @ wk.double().T) ** 2
+    ref_o = h[:N].double() @ wv.double().T
+    for got, ref, units in ((h, ref_h, 3), (out, ref_o, 1)):
+        assert torch.isnan(got[N]).all(), "a row past the end was written"
+        err = (got[:N].double() - ref).abs().max().item() / ref.abs().max().item()
+        assert err <= units * UNIT[dtype], err
+
+
+@pytest.mark.parametrize("N,C,F,E,k,r", [(100, 64, 64, 4, 2, 8), (700, 192, 320, 32, 4, 16), (2031, 1024, 1792, 8, 2, 32),
+                                         (5000, 128, 256, 16, 2, 8), (300, 2048, 1024, 16, 2, 32)])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_layer_with_adapter_columns_and_residual(device, dtype, N, C, F, E, k, r):
+    """The whole FUSED layer (adapter columns, K-extension, residual) against
+    float64 with the dtype's rounding of each stage bounded."""
+    import torch
+    from rwkv_mlx_amd.moe import build_layer
+    dt = {"f16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    torch.manual_seed(N + E)
+    m = build_layer(C, F, E, k, r).to(device=device, dtype=dt).requires_grad_(False)
+    m.base.x_k.uniform_(0, 1)
+    m.lora_A.normal_(0, C ** -0.5)
+    m.lora_B.normal_(0, 0.3)
+    x = torch.randn(1, N, C, device=device).to(dt)
+    res = torch.randn(1, N, C, device=device).to(dt)
+    ex = {}
+    with torch.no_grad():
+        out = m(x, residual=res, extras=ex)[0]
+        out2 = m(x, residual=res)[0]
+    assert torch.equal(out, out2)
+    xd = x.double()
+    sh = torch.cat([torch.zeros_like(xd[:, :1]), xd[:, :-1]], 1)
+    base = torch.relu((xd + (sh - xd) * m.base.x_k.double()) @ m.base.key.weight.double().T) ** 2 \
+        @ m.base.value.weight.double().T
+    w = torch.zeros(N, E, dtype=torch.float64, device=device).scatter(1, ex["inds"].long(), ex["gates"].double())
+    delta = sum(w[:, e:e + 1] * (xd[0] @ m.lora_A[e].double() @ m.lora_B[e].double()) for e in range(E))
+    ref = res.double() + base + delta
+    err = (out.double() - ref).norm().item() / ref.norm().item()
+    # the mix, h, U, the output and the residual sum each round to dtype
+    assert err <= 5 * UNIT[dtype], err
+
+
+@pytest.mark.parametrize("N,C,F,E,k,hot", [(3, 64, 64, 2, 1, False), (130, 128, 192, 64, 1, False),
+                                           (600, 64, 320, 8, 2, True), (3000, 256, 512, 16, 2, True),
+                                           (20000, 64, 64, 4, 1, True), (2500, 768, 768, 5, 3, False)])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_row_groups(device, dtype, N, C, F, E, k, hot):
+    """MoE_CMix's grouped products: groups that are empty, ragged, or hold
+    nearly every token, against the routed rows in float64."""
+    import torch
+    from rwkv_mlx_amd import MoE_CMix, RWKVConfig
+    dt = {"f16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    torch.manual_seed(N + E)
+    m = MoE_CMix(RWKVConfig(n_embd=C, dim_ffn=F), 0, E, k).to(device=device, dtype=dt).requires_grad_(False)
+    m.x_k.uniform_(0, 1)
+    m.expert_key.normal_(0, C ** -0.5)
+    m.expert_val.normal_(0, F ** -0.5)
+    if hot:
+        m.router.logit_bias = torch.tensor([20.0] + [0.0] * (E - 1), device=device)
+    x = torch.randn(1, N, C, device=device).to(dt)
+    ex = {}
+    with torch.no_grad():
+        out = m(x, extras=ex)[0][0].double()
+    xd = x[0].double()
+    mix = torch.cat([torch.zeros_like(xd[:1]), xd[:-1]]) - xd
+    ref = torch.zeros_like(xd)
+    w = torch.zeros(N, E, dtype=torch.float64, device=device).scatter(1, ex["inds"].long(), ex["gates"].double())
+    for e in range(E):
+        at = (ex["inds"] == e).any(1).nonzero()[:, 0]
+        y = torch.relu((xd[at] + mix[at] * m.x_k[e, 0, 0].double()) @ m.expert_key[e].double().T) ** 2 \
+            @ m.expert_val[e].double().T
+        ref = ref.index_add(0, at, w[at, e:e + 1] * y)
+    err = (out - ref).norm().item() / ref.norm().item()
+    assert np.isfinite(err) and err <= 5 * UNIT[dtype], err
