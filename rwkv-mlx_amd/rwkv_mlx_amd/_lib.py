@@ -8,6 +8,7 @@ if the library is missing, every call raises.
 from __future__ import annotations
 
 import ctypes
+from functools import lru_cache
 from pathlib import Path
 
 import torch
@@ -81,6 +82,9 @@ class Tensors(ctypes.Structure):
         "out", "losses", "logits", "inds", "gates", "gate_dense", "perm", "inv_perm", "offsets",
         "hidden", "base_out", "adapter_rows", "ortho_loss", "prepared", "prepared_base",
         "ln_weight", "ln_bias", "x_ln")]
+
+
+_TENSORS_SIZE = ctypes.sizeof(Tensors)
 
 
 class Grads(ctypes.Structure):
@@ -190,6 +194,28 @@ def make_desc(batch, seq_len, d_model, d_ffn, n_experts, top_k, lora_rank, dtype
     return Desc(batch, seq_len, d_model, d_ffn, n_experts, top_k, lora_rank, dtype, mode, flags)
 
 
+@lru_cache(maxsize=1024)
+def plan(entry: str, *dims) -> tuple[Desc, int]:
+    """The descriptor of make_desc(*dims) and the workspace that
+    ``rwkvmoe_<entry>workspace_bytes`` asks for it: a function of the sizes
+    alone, kept for calls that repeat them.  The descriptor is shared and only
+    read."""
+    desc = make_desc(*dims)
+    n = ctypes.c_size_t(0)
+    name = f"rwkvmoe_{entry}workspace_bytes"
+    st = getattr(lib(), name)(ctypes.byref(desc), ctypes.byref(n))
+    if st != 0:
+        raise RwkvMoeError(st, name)
+    return desc, int(n.value)
+
+
+@lru_cache(maxsize=1024)
+def plan_forward(*dims) -> tuple[Desc, int, bool]:
+    """plan("", *dims) and whether the forward reads prepared_base."""
+    desc, nbytes = plan("", *dims)
+    return desc, nbytes, reads_prepared_base(desc)
+
+
 def workspace_bytes(desc: Desc) -> int:
     n = ctypes.c_size_t(0)
     st = lib().rwkvmoe_workspace_bytes(ctypes.byref(desc), ctypes.byref(n))
@@ -259,9 +285,7 @@ def backward_workspace_bytes(desc: Desc) -> int:
 def backward(desc: Desc, ws, ws_bytes: int, stream, entry: str = "rwkvmoe_backward", **kw) -> None:
     """rwkvmoe_backward (or rwkvmoe_ortho_backward) with the named
     rwkvmoe_grads fields."""
-    g = Grads()
-    for k, v in kw.items():
-        setattr(g, k, ptr(v))
+    g = Grads(**{k: ptr(v) for k, v in kw.items()})
     st = getattr(lib(), entry)(ctypes.byref(desc), ctypes.byref(g), ptr(ws), ctypes.c_size_t(ws_bytes), stream)
     if st != 0:
         raise RwkvMoeError(st, entry)
@@ -277,9 +301,7 @@ def router_backward_workspace_bytes(desc: Desc) -> int:
 
 def router_backward(desc: Desc, ws, ws_bytes: int, stream, **kw) -> None:
     """rwkvmoe_router_backward with the named rwkvmoe_router_grads fields."""
-    g = RouterGrads()
-    for k, v in kw.items():
-        setattr(g, k, ptr(v))
+    g = RouterGrads(**{k: ptr(v) for k, v in kw.items()})
     st = lib().rwkvmoe_router_backward(ctypes.byref(desc), ctypes.byref(g), ptr(ws), ctypes.c_size_t(ws_bytes), stream)
     if st != 0:
         raise RwkvMoeError(st, "rwkvmoe_router_backward")
@@ -295,9 +317,7 @@ def layer_norm_backward_workspace_bytes(desc: Desc) -> int:
 
 def layer_norm_backward(desc: Desc, ws, ws_bytes: int, stream, **kw) -> None:
     """rwkvmoe_layer_norm_backward with the named rwkvmoe_ln_grads fields."""
-    g = LnGrads()
-    for k, v in kw.items():
-        setattr(g, k, ptr(v))
+    g = LnGrads(**{k: ptr(v) for k, v in kw.items()})
     st = lib().rwkvmoe_layer_norm_backward(ctypes.byref(desc), ctypes.byref(g), ptr(ws), ctypes.c_size_t(ws_bytes),
                                            stream)
     if st != 0:
@@ -314,9 +334,7 @@ def experts_backward_workspace_bytes(desc: Desc) -> int:
 
 def experts_backward(desc: Desc, ws, ws_bytes: int, stream, **kw) -> None:
     """rwkvmoe_experts_backward with the named rwkvmoe_experts_grads fields."""
-    g = ExpertsGrads()
-    for k, v in kw.items():
-        setattr(g, k, ptr(v))
+    g = ExpertsGrads(**{k: ptr(v) for k, v in kw.items()})
     st = lib().rwkvmoe_experts_backward(ctypes.byref(desc), ctypes.byref(g), ptr(ws), ctypes.c_size_t(ws_bytes),
                                         stream)
     if st != 0:
@@ -325,19 +343,16 @@ def experts_backward(desc: Desc, ws, ws_bytes: int, stream, **kw) -> None:
 
 def ptr(t) -> int | None:
     """Device address of a tensor (None for None)."""
-    if t is None:
-        return None
-    if isinstance(t, int):
+    if t is None or isinstance(t, int):
         return t
     return t.data_ptr()
 
 
-def make_tensors(**kw) -> Tensors:
-    t = Tensors()
-    t.struct_size = ctypes.sizeof(Tensors)
-    for k, v in kw.items():
-        setattr(t, k, ptr(v))
-    return t
+def make_tensors(*args, **kw) -> Tensors:
+    """rwkvmoe_tensors of the given tensors (or None), by position in the
+    struct's order or by name."""
+    return Tensors(_TENSORS_SIZE, *[None if v is None else ptr(v) for v in args],
+                   **{k: ptr(v) for k, v in kw.items() if v is not None})
 
 
 def forward_noalloc(desc: Desc, tensors: Tensors, stream) -> None:
@@ -349,8 +364,7 @@ def forward_noalloc(desc: Desc, tensors: Tensors, stream) -> None:
 
 def call(name: str, desc: Desc, tensors: Tensors, ws, ws_bytes: int, stream) -> None:
     """Invoke a stage entry point; raise RwkvMoeError on a non-zero status."""
-    fn = getattr(lib(), name)
-    st = fn(ctypes.byref(desc), ctypes.byref(tensors), ptr(ws), ctypes.c_size_t(ws_bytes), stream)
+    st = getattr(lib(), name)(ctypes.byref(desc), ctypes.byref(tensors), ptr(ws), ws_bytes, stream)
     if st != 0:
         raise RwkvMoeError(st, name)
 
@@ -405,4 +419,7 @@ class KernelTimer:
 
 
 def current_stream(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The hipStream_t of torch's current stream on `device` (without the
+    Stream object that torch.cuda.current_stream makes, 2.5 us a call)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)

@@ -51,8 +51,9 @@ class Workspace:
     def __init__(self):
         self._buf: dict[tuple, torch.Tensor] = {}
 
-    def get(self, device: torch.device, nbytes: int) -> torch.Tensor:
-        key = (device, torch.cuda.current_stream(device).cuda_stream)
+    def get(self, device: torch.device, nbytes: int, stream: int | None = None) -> torch.Tensor:
+        """`stream`: the current stream's handle, where the caller has it."""
+        key = (device, _lib.current_stream(device) if stream is None else stream)
         b = self._buf.get(key)
         if b is None or b.numel() < nbytes:
             b = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
@@ -61,6 +62,16 @@ class Workspace:
 
 
 _WS = Workspace()
+
+
+def operand(t: torch.Tensor, device: torch.device, dtype: torch.dtype) -> torch.Tensor:
+    """`t` detached, on `device`, in `dtype` and contiguous; `t` itself where it
+    is that already and has no gradient (a launch takes only its address)."""
+    if t.requires_grad:
+        t = t.detach()
+    if t.dtype is dtype and t.device == device and t.is_contiguous():
+        return t
+    return t.to(device=device, dtype=dtype).contiguous()
 
 
 class RWKV_CMix_x070(nn.Module):
@@ -92,20 +103,19 @@ class RWKV_CMix_x070(nn.Module):
         F = self.key.weight.shape[0]
         if B * T == 0:
             return torch.empty(B, T, C, dtype=dt, device=x.device)
+        dev = x.device
         x = x.to(dt).contiguous()
-        xk = self.x_k.detach().to(dt).reshape(C).contiguous()
-        wk = self.key.weight.detach().to(dt).contiguous()
-        wv = self.value.weight.detach().to(dt).contiguous()
+        xk = operand(self.x_k, dev, dt).reshape(C)
+        wk = operand(self.key.weight, dev, dt)
+        wv = operand(self.value.weight, dev, dt)
         flags = _lib.HAS_PREV if x_prev is not None else 0
-        desc = _lib.make_desc(B, T, C, F, 1, 1, 1, dt, _lib.MODE_FUSED, flags)
-        nbytes = _lib.workspace_bytes(desc)
-        ws = _WS.get(x.device, nbytes)
-        hidden = torch.empty(B * T, F, dtype=dt, device=x.device)
+        desc, nbytes = _lib.plan("", B, T, C, F, 1, 1, 1, dt, _lib.MODE_FUSED, flags)
+        stream = _lib.current_stream(dev)
+        ws = _WS.get(dev, nbytes, stream)
+        hidden = torch.empty(B * T, F, dtype=dt, device=dev)
         out = torch.empty_like(x)
-        xp = x_prev.to(device=x.device, dtype=dt).contiguous() if x_prev is not None else None
-        stream = _lib.current_stream(x.device)
-        t = _lib.make_tensors(x=x, x_prev=xp, x_k=xk, w_key=wk, hidden=hidden)
+        xp = operand(x_prev, dev, dt) if x_prev is not None else None
+        t = _lib.make_tensors(x=x, x_prev=xp, x_k=xk, w_key=wk, w_value=wv, hidden=hidden, base_out=out)
         _lib.call("rwkvmoe_cmix_key", desc, t, ws, nbytes, stream)
-        t = _lib.make_tensors(hidden=hidden, w_value=wv, base_out=out)
         _lib.call("rwkvmoe_cmix_value", desc, t, ws, nbytes, stream)
         return out

@@ -38,12 +38,13 @@ Differences, all deliberate:
 from __future__ import annotations
 
 import math
+from functools import lru_cache
 
 import torch
 from torch import nn
 
 from . import _lib
-from .model import _WS, RWKV_CMix_x070, RWKVConfig, require_device
+from .model import _WS, RWKV_CMix_x070, RWKVConfig, operand, require_device
 
 __all__ = ["Router", "LoRAMoE_CMix", "MoE_CMix", "RWKV_CMix_x070", "RWKVConfig", "channel_mixing_rnn"]
 
@@ -66,6 +67,7 @@ def _gate_plan(dt: torch.dtype, gate_dtype: torch.dtype):
     return torch.float32, _lib.GATE_F32
 
 
+@lru_cache(maxsize=256)
 def _dtype_plan(x_dtype, base_dtypes, gate_dtype, adapter_dtypes):
     """MLX promotion of LoRAMoE_CMix's operands onto the library's dtypes.
 
@@ -95,17 +97,18 @@ class _RouterFunction(torch.autograd.Function):
     def forward(ctx, x, wg, bias, dims):
         B, T, C, E, k, dt = dims
         flags = _lib.HAS_BIAS if bias is not None else 0
-        desc = _lib.make_desc(B, T, C, 64, E, k, 1, dt, _lib.MODE_FUSED, flags)
-        nbytes = _lib.workspace_bytes(desc)
-        ws = _WS.get(x.device, nbytes)
+        dims = (B, T, C, 64, E, k, 1, dt, _lib.MODE_FUSED, flags)
+        desc, nbytes = _lib.plan("", *dims)
+        stream = _lib.current_stream(x.device)
+        ws = _WS.get(x.device, nbytes, stream)
         inds = torch.empty(B, T, k, dtype=torch.int32, device=x.device)
         gates = torch.empty(B, T, k, dtype=dt, device=x.device)
         losses = torch.empty(2, dtype=torch.float32, device=x.device)
         logits = torch.empty(B * T, E, dtype=torch.float32, device=x.device)
         t = _lib.make_tensors(x=x, w_gate=wg, logit_bias=bias, inds=inds, gates=gates, losses=losses, logits=logits)
-        _lib.call("rwkvmoe_router_topk", desc, t, ws, nbytes, _lib.current_stream(x.device))
+        _lib.call("rwkvmoe_router_topk", desc, t, ws, nbytes, stream)
         ctx.save_for_backward(x, wg, logits, inds)
-        ctx.desc = desc
+        ctx.plan = dims
         ctx.mark_non_differentiable(inds)
         return inds, gates, losses
 
@@ -121,10 +124,10 @@ class _RouterFunction(torch.autograd.Function):
         if grads:
             dg = None if d_gates is None else d_gates.to(x.dtype).contiguous()
             dl = None if d_losses is None else d_losses.to(torch.float32).contiguous()
-            nbytes = _lib.router_backward_workspace_bytes(ctx.desc)
-            ws = _WS.get(x.device, nbytes)
-            _lib.router_backward(ctx.desc, ws, nbytes, _lib.current_stream(x.device), x=x, w_gate=wg, logits=logits,
-                                 inds=inds, d_gates=dg, d_losses=dl, **grads)
+            desc, nbytes = _lib.plan("router_backward_", *ctx.plan)
+            stream = _lib.current_stream(x.device)
+            _lib.router_backward(desc, _WS.get(x.device, nbytes, stream), nbytes, stream, x=x, w_gate=wg,
+                                 logits=logits, inds=inds, d_gates=dg, d_losses=dl, **grads)
         return grads.get("d_x"), grads.get("d_w_gate"), None, None
 
 
@@ -167,20 +170,21 @@ class Router(nn.Module):
                 (B, T, C, E, k, ct))
             return inds, gates.to(dt), losses[0], losses[1]  # gates in x's dtype (moe.py:86)
         x = x.contiguous()
-        gdt, flags = _gate_plan(dt, self.gate.weight.dtype)  # the gate as stored (moe.py:56)
-        wg = self.gate.weight.detach().to(device=x.device, dtype=gdt).contiguous()
+        weight = self.gate.weight
+        gdt, flags = _gate_plan(dt, weight.dtype)  # the gate as stored (moe.py:56)
+        wg = operand(weight, x.device, gdt)
         bias = self.logit_bias
         if bias is not None:
-            bias = bias.detach().to(device=x.device, dtype=torch.float32).contiguous()
+            bias = operand(bias, x.device, torch.float32)
             flags |= _lib.HAS_BIAS
-        desc = _lib.make_desc(B, T, C, 64, E, k, 1, dt, _lib.MODE_FUSED, flags)
-        nbytes = _lib.workspace_bytes(desc)
-        ws = _WS.get(x.device, nbytes)
+        desc, nbytes = _lib.plan("", B, T, C, 64, E, k, 1, dt, _lib.MODE_FUSED, flags)
+        stream = _lib.current_stream(x.device)
+        ws = _WS.get(x.device, nbytes, stream)
         inds = torch.empty(B, T, k, dtype=torch.int32, device=x.device)
         gates = torch.empty(B, T, k, dtype=dt, device=x.device)
         losses = torch.empty(2, dtype=torch.float32, device=x.device)
         t = _lib.make_tensors(x=x, w_gate=wg, logit_bias=bias, inds=inds, gates=gates, losses=losses)
-        _lib.call("rwkvmoe_router_topk", desc, t, ws, nbytes, _lib.current_stream(x.device))
+        _lib.call("rwkvmoe_router_topk", desc, t, ws, nbytes, stream)
         return inds, gates, losses[0], losses[1]
 
 
@@ -211,7 +215,7 @@ def _ln_fused_ok(x, w, b, eps, dt):
 
 def _run_forward(x, xp, xk, wk, wv, wg, A, Bm, bias, res, dims, mode, extras, dflags=0, odt=None, ln=None):
     """rwkvmoe_forward on prepared (dtype-converted, contiguous) operands.
-    Returns (out, losses (2,) fp32, desc); `extras` (a dict or None)
+    Returns (out, losses (2,) fp32); `extras` (a dict or None)
     receives the tensors it names (logits, inds, gates, x_ln) as optional
     outputs.  dflags: the dtype flags of a mixed layer (GATE_F32,
     ADAPTERS_F32), whose output dtype is odt.  ln: ln2's (weight, bias), run
@@ -219,16 +223,34 @@ def _run_forward(x, xp, xk, wk, wv, wg, A, Bm, bias, res, dims, mode, extras, df
     B, T, C, F, E, k, r, dt = dims
     flags = (_lib.HAS_PREV if xp is not None else 0) | (_lib.HAS_BIAS if bias is not None else 0) \
         | (_lib.ADD_RESIDUAL if res is not None else 0) | (_lib.LN_IN if ln is not None else 0) | dflags
-    desc = _lib.make_desc(B, T, C, F, E, k, r, dt, mode, flags)
-    nbytes = _lib.workspace_bytes(desc)
-    ws = _WS.get(x.device, nbytes)
+    desc, nbytes = _lib.plan("", B, T, C, F, E, k, r, dt, mode, flags)
+    stream = _lib.current_stream(x.device)
+    ws = _WS.get(x.device, nbytes, stream)
     out = torch.empty(x.shape, dtype=odt or x.dtype, device=x.device)
     losses = torch.empty(2, dtype=torch.float32, device=x.device)
     lnkw = dict(ln_weight=ln[0], ln_bias=ln[1]) if ln is not None else {}
     t = _lib.make_tensors(x=x, x_prev=xp, x_k=xk, w_key=wk, w_value=wv, w_gate=wg, lora_A=A, lora_B=Bm,
                           logit_bias=bias, residual=res, out=out, losses=losses, **lnkw, **(extras or {}))
-    _lib.call("rwkvmoe_forward", desc, t, ws, nbytes, _lib.current_stream(x.device))
-    return out, losses, desc
+    _lib.call("rwkvmoe_forward", desc, t, ws, nbytes, stream)
+    return out, losses
+
+
+def _two_losses(losses):
+    """(aux, z) of the (2,) buffer that a forward wrote, each a scalar tensor
+    of its own on that buffer's storage.  As outputs of an autograd node they
+    take their cotangents directly: indexing a (2,) output instead costs each
+    backward two zero fills, two copies and a sum."""
+    st = losses.untyped_storage()
+    return tuple(torch.empty((), dtype=losses.dtype, device=losses.device).set_(st, i, (), ()) for i in (0, 1))
+
+
+def _loss_cotangents(d_aux, d_z):
+    """The (2,) cotangent the library reads, None where neither loss has one."""
+    if d_aux is None and d_z is None:
+        return None
+    some = d_aux if d_aux is not None else d_z
+    zero = some.new_zeros(()) if d_aux is None or d_z is None else None
+    return torch.stack([zero if d is None else d for d in (d_aux, d_z)]).to(torch.float32)
 
 
 def _ln_backward(x, lnw, d_y, d_res, need_x, need_w, need_b, dims):
@@ -247,11 +269,10 @@ def _ln_backward(x, lnw, d_y, d_res, need_x, need_w, need_b, dims):
     if need_b:
         g["d_ln_bias"] = torch.empty_like(lnw)
     if g:
-        desc = _lib.make_desc(B, T, C, F, E, k, r, x.dtype)
-        nbytes = _lib.layer_norm_backward_workspace_bytes(desc)
-        ws = _WS.get(x.device, nbytes)
+        desc, nbytes = _lib.plan("layer_norm_backward_", B, T, C, F, E, k, r, x.dtype)
+        stream = _lib.current_stream(x.device)
         dr = d_res.to(x.dtype).contiguous() if need_x and d_res is not None else None
-        _lib.layer_norm_backward(desc, ws, nbytes, _lib.current_stream(x.device), x=x, ln_weight=lnw, d_y=d_y,
+        _lib.layer_norm_backward(desc, _WS.get(x.device, nbytes, stream), nbytes, stream, x=x, ln_weight=lnw, d_y=d_y,
                                  d_res=dr, **g)
     return g.get("d_x"), g.get("d_ln_weight"), g.get("d_ln_bias")
 
@@ -280,23 +301,24 @@ class _LoRAMoEFunction(torch.autograd.Function):
         if lnw is not None:  # ln2 in the layer's launches; LN(x) kept as the VJP's layer input
             ex["x_ln"] = torch.empty_like(x)
             ln = (lnw.detach(), lnb.detach())
-        out, losses, _ = _run_forward(x, xp, xk, wk, wv, wg, A, Bm, bias, res, dims, mode, ex, dflags, odt, ln)
+        out, losses = _run_forward(x, xp, xk, wk, wv, wg, A, Bm, bias, res, dims, mode, ex, dflags, odt, ln)
         xl = ex["x_ln"] if ln is not None else x
         ctx.save_for_backward(xl, A, Bm, wg, ex["logits"], ex["inds"], x if ln is not None else None, lnw)
         B, T, C, F, E, k, r, dt = dims
         if dflags:
-            ctx.desc = _lib.make_desc(B, T, C, F, E, k, r, torch.float32, mode, _lib.GATES_F16)
+            ctx.plan = (B, T, C, F, E, k, r, torch.float32, mode, _lib.GATES_F16)
         else:
-            ctx.desc = _lib.make_desc(B, T, C, F, E, k, r, dt, mode)
+            ctx.plan = (B, T, C, F, E, k, r, dt, mode)
+        ctx.set_materialize_grads(False)
         ctx.dims = (B, T, C, F, E, k, r)
         ctx.mixed = dflags != 0
         ctx.has_res = res is not None
         ctx.ln = ln is not None
         ctx.res_is_x = res_is_x and ln is not None and res is not None
-        return out, losses
+        return (out, *_two_losses(losses))
 
     @staticmethod
-    def backward(ctx, d_out, d_losses):
+    def backward(ctx, d_out, d_aux, d_z):
         x, A, Bm, wg, logits, inds, x0, lnw = ctx.saved_tensors
         need = ctx.needs_input_grad
         # x: the layer's input (LN(x0) with ln2); its cotangent feeds ln2's VJP
@@ -317,11 +339,11 @@ class _LoRAMoEFunction(torch.autograd.Function):
             d_out = torch.zeros(x.shape, dtype=cdt, device=x.device)
         if grads:
             dob = d_out.to(cdt).contiguous()
-            dl = None if d_losses is None else d_losses.to(torch.float32).contiguous()
-            nbytes = _lib.backward_workspace_bytes(ctx.desc)
-            ws = _WS.get(x.device, nbytes)
-            _lib.backward(ctx.desc, ws, nbytes, _lib.current_stream(x.device), x=xb, w_gate=wgb, lora_A=Ab, lora_B=Bb,
-                          logits=logits, inds=inds, d_out=dob, d_losses=dl, **grads)
+            dl = _loss_cotangents(d_aux, d_z)
+            desc, nbytes = _lib.plan("backward_", *ctx.plan)
+            stream = _lib.current_stream(x.device)
+            _lib.backward(desc, _WS.get(x.device, nbytes, stream), nbytes, stream, x=xb, w_gate=wgb, lora_A=Ab,
+                          lora_B=Bb, logits=logits, inds=inds, d_out=dob, d_losses=dl, **grads)
         d_x = grads.get("d_x")
         d_lnw = d_lnb = None
         fuse_res = ctx.res_is_x and need[0]  # x + ffn(ln2(x)): d_out joins d_x inside ln2's VJP
@@ -340,25 +362,30 @@ class _OrthoFunction(torch.autograd.Function):
     rwkvmoe_ortho_backward: d lora_A_i = 2 Σ_{j≠i} A_j (A_jᵀ A_i) · d_ortho."""
 
     @staticmethod
-    def forward(ctx, A, desc):
-        nbytes = _lib.workspace_bytes(desc)
-        ws = _WS.get(A.device, nbytes)
-        out = torch.empty(1, dtype=torch.float32, device=A.device)
-        t = _lib.make_tensors(lora_A=A, ortho_loss=out)
-        _lib.call("rwkvmoe_ortho_loss", desc, t, ws, nbytes, _lib.current_stream(A.device))
+    def forward(ctx, A, dims):
         ctx.save_for_backward(A)
-        ctx.desc = desc
-        return out
+        ctx.plan = dims
+        return _ortho_loss(A, dims)
 
     @staticmethod
     def backward(ctx, d):
         (A,) = ctx.saved_tensors
         dA = torch.empty_like(A)
-        nbytes = _lib.backward_workspace_bytes(ctx.desc)
-        ws = _WS.get(A.device, nbytes)
-        _lib.backward(ctx.desc, ws, nbytes, _lib.current_stream(A.device), entry="rwkvmoe_ortho_backward", lora_A=A,
-                      d_lora_A=dA, d_ortho=d.to(torch.float32).contiguous())
+        desc, nbytes = _lib.plan("backward_", *ctx.plan)
+        stream = _lib.current_stream(A.device)
+        _lib.backward(desc, _WS.get(A.device, nbytes, stream), nbytes, stream, entry="rwkvmoe_ortho_backward",
+                      lora_A=A, d_lora_A=dA, d_ortho=d.to(torch.float32).contiguous())
         return dA, None
+
+
+def _ortho_loss(A, dims):
+    """rwkvmoe_ortho_loss of a contiguous lora_A: an fp32 scalar."""
+    desc, nbytes = _lib.plan("", *dims)
+    stream = _lib.current_stream(A.device)
+    out = torch.empty((), dtype=torch.float32, device=A.device)
+    _lib.call("rwkvmoe_ortho_loss", desc, _lib.make_tensors(lora_A=A, ortho_loss=out),
+              _WS.get(A.device, nbytes, stream), nbytes, stream)
+    return out
 
 
 class _SourceKey:
@@ -372,17 +399,22 @@ class _SourceKey:
 
     def __init__(self, params, extra):
         self.alias = tuple(p.detach() for p in params)
-        self.state = tuple((p._version, p.dtype, tuple(p.shape)) for p in params)
+        self.state = tuple((p._version, p.dtype) for p in params)
         self.extra = extra
 
     def matches(self, params, extra) -> bool:
         if extra != self.extra or len(params) != len(self.alias):
             return False
         for p, a, st in zip(params, self.alias, self.state):
-            if (p.untyped_storage().data_ptr() != a.untyped_storage().data_ptr() or p.data_ptr() != a.data_ptr()
-                    or (p._version, p.dtype, tuple(p.shape)) != st):
+            # (is_set_to: the same storage, offset, shape and strides)
+            if p._version != st[0] or p.dtype is not st[1] or not p.is_set_to(a):
                 return False
         return True
+
+
+class _OnlyLN(dict):
+    """The `extras` of a call that wants x_ln alone (an RNN-mode step with ln2:
+    its next state), so that the routing is not written out for it."""
 
 
 class LoRAMoE_CMix(nn.Module):
@@ -452,17 +484,19 @@ class LoRAMoE_CMix(nn.Module):
         (the base is always detached: stop_gradient).  Returns (dt, flags,
         out_dt, [x_k, W_key, W_value, W_gate, lora_A, lora_B])."""
         base = self.base
-        params = [base.x_k, base.key.weight, base.value.weight, self.router.gate.weight, self.lora_A, self.lora_B]
-        dt, gdt, adt, flags, odt = _dtype_plan(x.dtype, [p.dtype for p in params[:3]], params[3].dtype,
-                                               [params[4].dtype, params[5].dtype])
+        xk, wk, wv, wg, A, Bm = params = (base.x_k, base.key.weight, base.value.weight, self.router.gate.weight,
+                                          self.lora_A, self.lora_B)
+        dt, gdt, adt, flags, odt = _dtype_plan(x.dtype, (xk.dtype, wk.dtype, wv.dtype), wg.dtype,
+                                               (A.dtype, Bm.dtype))
         if uniform:
             dt = gdt = adt = odt = _promote(x.dtype, *[p.dtype for p in params])
             flags = 0
-        want = [dt, dt, dt, gdt, adt, adt]
-        ops = [(p if differentiable and i >= 3 else p.detach()).to(device=x.device, dtype=want[i]).contiguous()
-               for i, p in enumerate(params)]
-        ops[0] = ops[0].reshape(-1)
-        return dt, flags, odt, ops
+        dev = x.device
+        if differentiable:
+            wg, A, Bm = [p.to(device=dev, dtype=d).contiguous() for p, d in ((wg, gdt), (A, adt), (Bm, adt))]
+        else:
+            wg, A, Bm = operand(wg, dev, gdt), operand(A, dev, adt), operand(Bm, dev, adt)
+        return dt, flags, odt, (operand(xk, dev, dt).reshape(-1), operand(wk, dev, dt), operand(wv, dev, dt), wg, A, Bm)
 
     def forward(self, x: torch.Tensor, x_prev: torch.Tensor | None = None,
                 residual: torch.Tensor | None = None, mode: str | None = None,
@@ -517,54 +551,47 @@ class LoRAMoE_CMix(nn.Module):
             return (out if residual is None else residual.to(odt) + out), nan, nan.clone()
         F = wk.shape[0]
         E, k, r = self.n_experts, self.top_k, self.lora_rank
-        if train:
-            xp = x_prev.detach().to(device=x.device, dtype=dt).contiguous() if x_prev is not None else None
-            bias = self.router.logit_bias
-            if bias is not None:
-                bias = bias.detach().to(device=x.device, dtype=torch.float32).contiguous()
-            res = residual.to(dt).contiguous() if residual is not None else None
-            out, losses = _LoRAMoEFunction.apply(x.to(dt).contiguous(), A, Bm, wg, xk, wk, wv, bias, xp, res,
-                                                 (B, T, C, F, E, k, r, dt), mode or self.mode, pflags, odt, lnw, lnb,
-                                                 residual is x)
-            return out, losses[0], losses[1]
-        x = x.to(dt).contiguous()
+        dev = x.device
         flags = pflags | (_lib.LN_IN if lnw is not None else 0)
-        xp = None
+        xp = res = None
         if x_prev is not None:
-            xp = x_prev.to(device=x.device, dtype=dt).contiguous()
+            xp = operand(x_prev, dev, dt)
             flags |= _lib.HAS_PREV
         bias = self.router.logit_bias
         if bias is not None:
-            bias = bias.detach().to(device=x.device, dtype=torch.float32).contiguous()
+            bias = operand(bias, dev, torch.float32)
             flags |= _lib.HAS_BIAS
-        res = None
+        if train:
+            res = residual.to(dt).contiguous() if residual is not None else None
+            return _LoRAMoEFunction.apply(x.to(dt).contiguous(), A, Bm, wg, xk, wk, wv, bias, xp, res,
+                                          (B, T, C, F, E, k, r, dt), mode or self.mode, pflags, odt, lnw, lnb,
+                                          residual is x)
+        x = x.to(dt).contiguous()
         if residual is not None:
             res = residual.to(dt).contiguous()  # in x's dtype; added to the output in out's dtype
             flags |= _lib.ADD_RESIDUAL
-        desc = _lib.make_desc(B, T, C, F, E, k, r, dt, mode or self.mode, flags)
-        nbytes = _lib.workspace_bytes(desc)
-        ws = _WS.get(x.device, nbytes)
-        out = torch.empty(B, T, C, dtype=odt, device=x.device)
-        losses = torch.empty(2, dtype=torch.float32, device=x.device)
+        desc, nbytes, reads_base = _lib.plan_forward(B, T, C, F, E, k, r, dt, mode or self.mode, flags)
+        stream = _lib.current_stream(dev)
+        ws = _WS.get(dev, nbytes, stream)
+        out = torch.empty(B, T, C, dtype=odt, device=dev)
+        losses = torch.empty(2, dtype=torch.float32, device=dev)
         kw = {}
         if extras is not None:
-            kw = {"inds": torch.empty(B * T, k, dtype=torch.int32, device=x.device),
-                  "gates": torch.empty(B * T, k, dtype=dt, device=x.device),
-                  "logits": torch.empty(B * T, E, dtype=torch.float32, device=x.device)}
+            if not isinstance(extras, _OnlyLN):
+                kw = {"inds": torch.empty(B * T, k, dtype=torch.int32, device=dev),
+                      "gates": torch.empty(B * T, k, dtype=dt, device=dev),
+                      "logits": torch.empty(B * T, E, dtype=torch.float32, device=dev)}
             if lnw is not None:
-                kw["x_ln"] = torch.empty(B, T, C, dtype=dt, device=x.device)
-        if lnw is not None:
-            kw.update(ln_weight=lnw, ln_bias=lnb)
+                kw["x_ln"] = torch.empty(B, T, C, dtype=dt, device=dev)
         prep = self._prepared(A, Bm, dt, flags)
         # decode-sized calls read the base weights in the decode launches' layout
         # (laid out only when this forward reads them)
-        pbase = self._prepared_base(wk, wv, dt) if _lib.reads_prepared_base(desc) else None
-        t = _lib.make_tensors(x=x, x_prev=xp, x_k=xk, w_key=wk, w_value=wv, w_gate=wg, lora_A=A, lora_B=Bm,
-                              logit_bias=bias, residual=res, out=out, losses=losses, prepared=prep,
-                              prepared_base=pbase, **kw)
-        _lib.call("rwkvmoe_forward", desc, t, ws, nbytes, _lib.current_stream(x.device))
+        pbase = self._prepared_base(wk, wv, dt) if reads_base else None
+        t = _lib.make_tensors(x, xp, xk, wk, wv, wg, A, Bm, bias, res, out, losses, prepared=prep,
+                              prepared_base=pbase, ln_weight=lnw, ln_bias=lnb, **kw)
+        _lib.call("rwkvmoe_forward", desc, t, ws, nbytes, stream)
         if extras is not None:
-            extras.update({n: v for n, v in kw.items() if n not in ("ln_weight", "ln_bias")})
+            extras.update(kw)
         return out, losses[0], losses[1]
 
     def decode_step(self, x: torch.Tensor, x_prev: torch.Tensor, ln=None):
@@ -576,7 +603,7 @@ class LoRAMoE_CMix(nn.Module):
         if ln is None:
             out, aux, z = self.forward(x.unsqueeze(1), x_prev=x_prev)
             return out.squeeze(1), aux, z, x
-        ex = {}
+        ex = _OnlyLN()
         out, aux, z = self.forward(x.unsqueeze(1), x_prev=x_prev, extras=ex, ln=ln)
         return out.squeeze(1), aux, z, ex["x_ln"].reshape(x.shape)
 
@@ -586,17 +613,10 @@ class LoRAMoE_CMix(nn.Module):
         A = self.lora_A
         require_device(A, "orthogonal_loss")
         E, C, r = A.shape
-        dt = A.dtype
-        desc = _lib.make_desc(1, 1, C, 64, E, 1, r, dt)
+        dims = (1, 1, C, 64, E, 1, r, A.dtype)
         if torch.is_grad_enabled() and A.requires_grad:
-            return _OrthoFunction.apply(A.contiguous(), desc)[0]
-        A = A.detach().contiguous()
-        nbytes = _lib.workspace_bytes(desc)
-        ws = _WS.get(A.device, nbytes)
-        out = torch.empty(1, dtype=torch.float32, device=A.device)
-        t = _lib.make_tensors(lora_A=A, ortho_loss=out)
-        _lib.call("rwkvmoe_ortho_loss", desc, t, ws, nbytes, _lib.current_stream(A.device))
-        return out[0]
+            return _OrthoFunction.apply(A.contiguous(), dims)
+        return _ortho_loss(A.detach().contiguous(), dims)
 
 
 class _ExpertsFunction(torch.autograd.Function):
@@ -611,9 +631,9 @@ class _ExpertsFunction(torch.autograd.Function):
         N = B * T
         flags = (_lib.HAS_PREV if xp is not None else 0) | (_lib.HAS_BIAS if bias is not None else 0) | (
             _lib.ADD_RESIDUAL if res is not None else 0) | (_lib.LN_IN if lnw is not None else 0)
-        desc = _lib.make_desc(B, T, C, F, E, k, 1, dt, _lib.MODE_FUSED, flags)
-        nbytes = _lib.experts_workspace_bytes(desc)
-        ws = _WS.get(x.device, nbytes)
+        desc, nbytes = _lib.plan("experts_", B, T, C, F, E, k, 1, dt, _lib.MODE_FUSED, flags)
+        stream = _lib.current_stream(x.device)
+        ws = _WS.get(x.device, nbytes, stream)
         out = torch.empty_like(x)
         losses = torch.empty(2, dtype=torch.float32, device=x.device)
         logits = torch.empty(N, E, dtype=torch.float32, device=x.device)
@@ -623,18 +643,19 @@ class _ExpertsFunction(torch.autograd.Function):
             lnkw = dict(ln_weight=lnw.detach(), ln_bias=lnb.detach(), x_ln=torch.empty_like(x))
         t = _lib.make_tensors(x=x, x_prev=xp, x_k=xk, w_key=wk, w_value=wv, w_gate=wg, logit_bias=bias,
                               residual=res, out=out, losses=losses, logits=logits, inds=inds, **lnkw)
-        _lib.call("rwkvmoe_experts_forward", desc, t, ws, nbytes, _lib.current_stream(x.device))
+        _lib.call("rwkvmoe_experts_forward", desc, t, ws, nbytes, stream)
         xl = lnkw["x_ln"] if lnw is not None else x
         ctx.save_for_backward(xl, xp, xk, wk, wv, wg, logits, inds, x if lnw is not None else None, lnw)
-        ctx.desc = _lib.make_desc(B, T, C, F, E, k, 1, dt, _lib.MODE_FUSED, flags & ~_lib.LN_IN)
+        ctx.plan = (B, T, C, F, E, k, 1, dt, _lib.MODE_FUSED, flags & ~_lib.LN_IN)
+        ctx.set_materialize_grads(False)
         ctx.dims = (B, T, C, F, E, k, 1)
         ctx.has_res = res is not None
         ctx.ln = lnw is not None
         ctx.res_is_x = res_is_x and lnw is not None and res is not None
-        return out, losses
+        return (out, *_two_losses(losses))
 
     @staticmethod
-    def backward(ctx, d_out, d_losses):
+    def backward(ctx, d_out, d_aux, d_z):
         x, xp, xk, wk, wv, wg, logits, inds, x0, lnw = ctx.saved_tensors
         need = ctx.needs_input_grad
         # x: the layer's input (LN(x0) with ln2); its cotangent feeds ln2's VJP
@@ -648,10 +669,10 @@ class _ExpertsFunction(torch.autograd.Function):
             d_out = torch.zeros_like(x)
         if grads:
             d_out = d_out.to(x.dtype).contiguous()
-            dl = None if d_losses is None else d_losses.to(torch.float32).contiguous()
-            nbytes = _lib.experts_backward_workspace_bytes(ctx.desc)
-            ws = _WS.get(x.device, nbytes)
-            _lib.experts_backward(ctx.desc, ws, nbytes, _lib.current_stream(x.device), x=x, x_prev=xp, x_k=xk,
+            dl = _loss_cotangents(d_aux, d_z)
+            desc, nbytes = _lib.plan("experts_backward_", *ctx.plan)
+            stream = _lib.current_stream(x.device)
+            _lib.experts_backward(desc, _WS.get(x.device, nbytes, stream), nbytes, stream, x=x, x_prev=xp, x_k=xk,
                                   w_key=wk, w_value=wv, w_gate=wg, logits=logits, inds=inds, d_out=d_out,
                                   d_losses=dl, **grads)
         d_x = grads.get("d_x")
@@ -715,7 +736,8 @@ class MoE_CMix(nn.Module):
             or (residual is not None and residual.requires_grad)
             or (lnp is not None and (lnp[0].requires_grad or lnp[1].requires_grad)))
         if not train:
-            return self._forward_nograd(x, x_prev, residual, extras, ln)
+            run = self._forward_nograd if torch.is_grad_enabled() else self._run
+            return run(x, x_prev, residual, extras, ln)
         E, k = self.n_experts, self.top_k
         params = [self.x_k, self.expert_key, self.expert_val, self.router.gate.weight]
         dt = _promote(x.dtype, *[p.dtype for p in params])  # one dtype: the backward has no fp32-gate form
@@ -734,9 +756,8 @@ class MoE_CMix(nn.Module):
         if bias is not None:
             bias = bias.detach().to(device=x.device, dtype=torch.float32).contiguous()
         res = residual.to(dt).contiguous() if residual is not None else None
-        out, losses = _ExpertsFunction.apply(x.to(dt).contiguous(), xp, xk, wk, wv, wg, bias, res,
-                                             (B, T, C, F, E, k, dt), lnw, lnb, residual is x)
-        return out, losses[0], losses[1]
+        return _ExpertsFunction.apply(x.to(dt).contiguous(), xp, xk, wk, wv, wg, bias, res,
+                                      (B, T, C, F, E, k, dt), lnw, lnb, residual is x)
 
     def _run(self, x, x_prev, residual, extras, ln=None):
         if x.dim() != 3:
@@ -755,45 +776,45 @@ class MoE_CMix(nn.Module):
                 return self._run(xn, x_prev, residual, extras)
             lnw = lnw.detach().to(device=x.device).contiguous()
             lnb = lnb.detach().to(device=x.device).contiguous()
-        gdt, gflags = _gate_plan(dt, self.router.gate.weight.dtype)  # the gate as stored (moe.py:56)
-        xk, wk, wv = [p.detach().to(device=x.device, dtype=dt).contiguous() for p in params]
-        wg = self.router.gate.weight.detach().to(device=x.device, dtype=gdt).contiguous()
+        dev = x.device
+        gate = self.router.gate.weight
+        gdt, gflags = _gate_plan(dt, gate.dtype)  # the gate as stored (moe.py:56)
+        xk, wk, wv = [operand(p, dev, dt) for p in params]
+        wg = operand(gate, dev, gdt)
         xk = xk.reshape(E, C)
         F = wk.shape[1]
         if B * T == 0:
-            nan = torch.full((), float("nan"), dtype=torch.float32, device=x.device)
-            out = torch.empty(B, T, C, dtype=dt, device=x.device)
+            nan = torch.full((), float("nan"), dtype=torch.float32, device=dev)
+            out = torch.empty(B, T, C, dtype=dt, device=dev)
             return (out if residual is None else residual.to(dt) + out), nan, nan.clone()
         x = x.to(dt).contiguous()
         flags = gflags | (_lib.LN_IN if lnw is not None else 0)
-        xp = None
+        xp = bias = res = None
         if x_prev is not None:
-            xp = x_prev.to(device=x.device, dtype=dt).contiguous()
+            xp = operand(x_prev, dev, dt)
             flags |= _lib.HAS_PREV
-        bias = self.router.logit_bias
-        if bias is not None:
-            bias = bias.detach().to(device=x.device, dtype=torch.float32).contiguous()
+        if self.router.logit_bias is not None:
+            bias = operand(self.router.logit_bias, dev, torch.float32)
             flags |= _lib.HAS_BIAS
-        res = None
         if residual is not None:
             res = residual.to(dt).contiguous()
             flags |= _lib.ADD_RESIDUAL
-        desc = _lib.make_desc(B, T, C, F, E, k, 1, dt, _lib.MODE_FUSED, flags)
-        nbytes = _lib.experts_workspace_bytes(desc)
-        ws = _WS.get(x.device, nbytes)
+        desc, nbytes = _lib.plan("experts_", B, T, C, F, E, k, 1, dt, _lib.MODE_FUSED, flags)
+        stream = _lib.current_stream(dev)
+        ws = _WS.get(dev, nbytes, stream)
         out = torch.empty_like(x)
-        losses = torch.empty(2, dtype=torch.float32, device=x.device)
+        losses = torch.empty(2, dtype=torch.float32, device=dev)
         kw = {}
         if extras is not None:
-            kw = {"inds": torch.empty(B * T, k, dtype=torch.int32, device=x.device),
-                  "gates": torch.empty(B * T, k, dtype=dt, device=x.device),
-                  "logits": torch.empty(B * T, E, dtype=torch.float32, device=x.device)}
+            if not isinstance(extras, _OnlyLN):
+                kw = {"inds": torch.empty(B * T, k, dtype=torch.int32, device=dev),
+                      "gates": torch.empty(B * T, k, dtype=dt, device=dev),
+                      "logits": torch.empty(B * T, E, dtype=torch.float32, device=dev)}
             if lnw is not None:
-                kw["x_ln"] = torch.empty(B, T, C, dtype=dt, device=x.device)
-        lnkw = dict(ln_weight=lnw, ln_bias=lnb) if lnw is not None else {}
-        t = _lib.make_tensors(x=x, x_prev=xp, x_k=xk, w_key=wk, w_value=wv, w_gate=wg, logit_bias=bias,
-                              residual=res, out=out, losses=losses, **kw, **lnkw)
-        _lib.call("rwkvmoe_experts_forward", desc, t, ws, nbytes, _lib.current_stream(x.device))
+                kw["x_ln"] = torch.empty(B, T, C, dtype=dt, device=dev)
+        t = _lib.make_tensors(x, xp, xk, wk, wv, wg, None, None, bias, res, out, losses, ln_weight=lnw, ln_bias=lnb,
+                              **kw)
+        _lib.call("rwkvmoe_experts_forward", desc, t, ws, nbytes, stream)
         if extras is not None:
             extras.update(kw)
         return out, losses[0], losses[1]
@@ -828,7 +849,7 @@ def channel_mixing_rnn(x: torch.Tensor, x_prev: torch.Tensor, ffn: nn.Module, ln
         if ln is None:
             out = ffn(xb, x_prev=pb)[0]
             return out.reshape(x.shape), x
-        ex = {}
+        ex = _OnlyLN()
         out = ffn(xb, x_prev=pb, extras=ex, ln=ln)[0]
         return out.reshape(x.shape), ex["x_ln"].reshape(x.shape)
     if isinstance(ffn, RWKV_CMix_x070):
