@@ -513,6 +513,8 @@ struct BwdLayout {
   size_t sgd, emask, pa, pb, pw;
   bool fx;  // the fused routing kernel computes S and G
   bool px;  // per-expert token contractions (else the dense products)
+  bool dx32;  // fp32, few tokens: bwd_f32.hip's products on the operands as stored
+  bool ox;    // the orthogonality gradient in bwd_f32.hip's two launches
   BwdExpertPlan xp;
   int np, ep;
 };
@@ -532,8 +534,10 @@ BwdLayout bwd_layout(const Dims& d) {
   const size_t s = d.s, np = L.np, ep = L.ep, kx = d.kx, C = d.C, N = d.N;
   L.fx = bwd_route_fuses(d.dtype, d.kx, d.C);
   L.px = d.dtype != 0;
+  L.dx32 = bwd_f32_direct(d.dtype, d.N, d.C, d.E, d.r);
+  L.ox = ortho_backward_direct(d.dtype, d.E, d.C, d.r);
   const size_t sg = L.fx ? 0 : 1;     // S and G in memory
-  const size_t dense = L.px ? 0 : 1;  // the dense token-contracted products
+  const size_t dense = L.px || L.dx32 ? 0 : 1;  // the dense token-contracted products
   const size_t px = L.px ? 1 : 0;
   L.at = take(kx * C * s);
   L.a_t = take(C * kx * s);
@@ -550,12 +554,12 @@ BwdLayout bwd_layout(const Dims& d) {
   L.sgdT = take(dense * kx * np * s);
   L.o = take(C * (kx + ep) * s);
   L.xp = bwd_expert_plan(d.N, d.C, d.E, d.k);
-  L.sgd = take(px * N * kx * s);
+  L.sgd = take((L.px || L.dx32 ? 1 : 0) * N * kx * s);
   L.emask = take(px * N * sizeof(unsigned long long));
   L.pa = take(px * (size_t)d.E * L.xp.R * C * d.r * sizeof(float));
   L.pb = take(px * (size_t)d.E * L.xp.R * C * d.r * sizeof(float));
   L.pw = take(px * (size_t)L.xp.RW * d.E * C * sizeof(float));
-  L.gram = take(kx * kx * s);
+  L.gram = take(std::max(L.ox ? ortho_gram_bytes(d.E, d.r) : 0, kx * kx * s));
   size_t sk = gemm_nt_partial_bytes(d.dtype, d.N, d.kx, d.C, GEMM_HINT_NO_SPLIT);
   sk = std::max(sk, gemm_nt_partial_bytes(d.dtype, d.C, d.kx + L.ep, L.np));
   sk = std::max(sk, gemm_nt_partial_bytes(d.dtype, d.N, d.C, d.kx + L.ep));
@@ -598,6 +602,21 @@ int backward_impl(const rwkvmoe_desc* desc, const rwkvmoe_grads* g, void* ws, si
   // B_rows in fragment order for the fused routing kernel; and the
   // per-expert selection counts
   int* cnt = (int*)(w + L.cnt);
+  if (L.dx32) {
+    const float* x = (const float*)g->x;
+    const float* dO = (const float*)g->d_out;
+    const float* A = (const float*)g->lora_A;
+    float* sgd = (float*)(w + L.sgd);
+    HIPTRY(launch_bwd_f32_first(x, dO, A, (const float*)g->lora_B, g->inds, N, C, E, d.k, d.r, kx, (float*)(w + L.S),
+                                (float*)(w + L.G), cnt, s));
+    HIPTRY(launch_bwd_route(dt, g->logits, g->inds, w + L.S, w + L.G, cnt, g->d_losses, N, E, d.k, d.r, kx, ep, np,
+                            w + L.dsd, w + L.dl, nullptr, nullptr, sgd, nullptr, s,
+                            (d.flags & RWKVMOE_GATES_F16) != 0));
+    HIPTRY(launch_bwd_f32_last(x, dO, A, (const float*)g->w_gate, (const float*)(w + L.dsd), sgd,
+                               (const float*)(w + L.dl), N, C, E, d.r, kx, ep, (float*)g->d_x, (float*)g->d_lora_A,
+                               (float*)g->d_lora_B, (float*)g->d_w_gate, s));
+    return RWKVMOE_OK;
+  }
   HIPTRY(launch_bwd_prep(dt, g->lora_A, g->lora_B, g->w_gate, E, C, d.r, kx, ep, fused, w + L.at, w + L.a_t,
                          w + L.b_rows, w + L.wgt, g->inds, N * d.k, cnt, s));
   unsigned long long* emask = L.px ? (unsigned long long*)(w + L.emask) : nullptr;
@@ -941,6 +960,10 @@ int ortho_backward_impl(const rwkvmoe_desc* desc, const rwkvmoe_grads* g, void* 
   hipStream_t s = (hipStream_t)stream;
   char* w = (char*)ws;
   const int dt = d.dtype, C = d.C, E = d.E, kx = d.kx;
+  if (L.ox) {
+    HIPTRY(launch_ortho_backward(dt, g->lora_A, E, C, d.r, g->d_ortho, (float*)(w + L.gram), g->d_lora_A, s));
+    return RWKVMOE_OK;
+  }
   float* part = (float*)(w + L.splitk);
   // A_all and A_T only
   HIPTRY(launch_bwd_prep(dt, g->lora_A, nullptr, nullptr, E, C, d.r, kx, L.ep, false, w + L.at, w + L.a_t, nullptr,

@@ -18,6 +18,7 @@
 // (transpose_pad_kernel: token-contiguous rows, zero-padded to Np tokens).
 #include <algorithm>
 
+#include "bwd.h"
 #include "common.h"
 #include "internal.h"
 
@@ -82,29 +83,10 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(const T* __restrict__ A, 
                                                        int frag, T* __restrict__ a_all, T* __restrict__ a_t,
                                                        T* __restrict__ b_rows, T* __restrict__ wgt,
                                                        const int* __restrict__ inds, int nk, int* __restrict__ cnt) {
-  // workgroup 0 (when cnt is given; dispatched first, so it overlaps the
-  // rest): tokens routed to each expert (the counts f_e of the aux loss,
-  // moe.py:80-83), 32 loads per thread in flight, LDS integer atomics
+  // workgroup 0 (when cnt is given; dispatched first, so it overlaps the rest)
   if (cnt && blockIdx.x == 0) {
     __shared__ int h[64];
-    if (threadIdx.x < 64) h[threadIdx.x] = 0;
-    __syncthreads();
-    const __amdgpu_buffer_rsrc_t ri = buf_rsrc(inds, (unsigned)nk * 4);
-    for (int b0 = 0; b0 < nk; b0 += 256 * 32) {
-      unsigned v[32];
-#pragma unroll
-      for (int u = 0; u < 32; ++u) {
-        const int j = b0 + u * 256 + (int)threadIdx.x;
-        v[u] = buf_load4(ri, j < nk ? (unsigned)j * 4u : kOOB);
-      }
-#pragma unroll
-      for (int u = 0; u < 32; ++u) {
-        const int j = b0 + u * 256 + (int)threadIdx.x, e = (int)v[u];
-        if (j < nk && e >= 0 && e < E) atomicAdd(&h[e], 1);
-      }
-    }
-    __syncthreads();
-    if ((int)threadIdx.x < E) cnt[threadIdx.x] = h[threadIdx.x];
+    count_selections(inds, nk, E, h, cnt);
     return;
   }
   const size_t i = (blockIdx.x - (cnt ? 1 : 0)) * (size_t)256 + threadIdx.x;
@@ -172,10 +154,10 @@ constexpr int kBwdMaxK = 8;
 // with P = softmax(ℓ), lse = log Σ exp ℓ, f = counts / (N k); the 8 threads
 // of a token each compute the gates (in slot order, as the forward does),
 // thread j takes slot j's dot product, and every 8th expert's terms, combined
-// with shuffles.  Then, in 64-column chunks: DSd = g·G and SGd = g·S on the
-// selected experts' columns (0 elsewhere), written row-major (DSd, tokens
-// < N) and, through an LDS tile, transposed with 16-byte stores (DSdᵀ, SGdᵀ;
-// zero for padding tokens N..Np-1).  dℓ goes out row-major (N x ep) and
+// with shuffles.  Then DSd = g·G and SGd = g·S on the selected experts'
+// columns (0 elsewhere), written row-major (tokens < N) and, where rT is given,
+// in 64-column chunks through an LDS tile transposed with 16-byte stores (DSdᵀ,
+// SGdᵀ; zero for padding tokens N..Np-1).  dℓ goes out row-major (N x ep) and
 // transposed into the rows kx..kx+ep-1 of the same transposed array as DSdᵀ.
 template <typename T>
 __global__ __launch_bounds__(kRouteThreads) void bwd_route_kernel(
@@ -190,6 +172,7 @@ __global__ __launch_bounds__(kRouteThreads) void bwd_route_kernel(
   __shared__ int ids[kRouteTok][kBwdMaxK], cnts[64];
   __shared__ float gs[kRouteTok][kBwdMaxK], gts[kRouteTok][kBwdMaxK], dgs[kRouteTok][kBwdMaxK];
   __shared__ int es[kRouteTok][kBwdMaxK];
+  __shared__ float gd[kRouteTok][65];  // gate of each expert (0: not selected)
   __shared__ T tD[64][kRouteTok + VEC], tS[64][kRouteTok + VEC];
   const int t0 = blockIdx.x * kRouteTok, tid = threadIdx.x;
   const int tl = tid >> 3, sub = tid & 7, t = t0 + tl;
@@ -233,6 +216,7 @@ __global__ __launch_bounds__(kRouteThreads) void bwd_route_kernel(
         if (e >= 0) {
           const T* sr = Sb + (size_t)tl * kx + e * r;
           const T* gr = Gb + (size_t)tl * kx + e * r;
+#pragma unroll 8
           for (int i = 0; i < r; ++i) acc += to_f(sr[i]) * to_f(gr[i]);
         }
         es[tl][sub] = e;
@@ -288,25 +272,52 @@ __global__ __launch_bounds__(kRouteThreads) void bwd_route_kernel(
     }
   }
   __syncthreads();
-  // DSd / SGd in 64-column chunks
-  for (int c0 = 0; c0 < kx; c0 += 64) {
+  for (int e = sub; e < 64; e += 8) {
+    float g = 0.f;
+    for (int j = 0; j < kBwdMaxK; ++j)
+      if (es[tl][j] == e) g = gs[tl][j];
+    gd[tl][e] = g;
+  }
+  __syncthreads();
+  // DSd and SGd of one 16-byte chunk (zero past token N and column E·r)
+  const float inv_r = 1.f / (float)r;
+  auto scaled = [&](int rl, int col0, Chunk<T>& od, Chunk<T>& os) {
+    Chunk<T> cs, cg;
+    cs.raw = cg.raw = zero4();
+    if (t0 + rl < N) {
+      cs.raw = *(const u32x4*)(Sb + (size_t)rl * kx + col0);
+      cg.raw = *(const u32x4*)(Gb + (size_t)rl * kx + col0);
+    }
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      const int col = col0 + j;
+      const int e = (int)(((float)col + 0.5f) * inv_r);  // col / r (col < 2^12)
+      const float g = col < E * r ? gd[rl][e] : 0.f;
+      od.e[j] = from_f<T>(g * to_f(cg.e[j]));
+      os.e[j] = from_f<T>(g * to_f(cs.e[j]));
+    }
+  };
+  if (!rT) {
+    // row-major only: every chunk by itself
+    const int cpr = kx / VEC;
+#pragma unroll 4
+    for (int i = tid; i < kRouteTok * cpr; i += NT) {
+      const int rl = i / cpr, col0 = (i - rl * cpr) * VEC, tt = t0 + rl;
+      if (tt >= N) continue;
+      Chunk<T> od, os;
+      scaled(rl, col0, od, os);
+      *(u32x4*)(dsd + (size_t)tt * kx + col0) = od.raw;
+      if (sgd) *(u32x4*)(sgd + (size_t)tt * kx + col0) = os.raw;
+    }
+  }
+  // in 64-column chunks, transposed through LDS too
+  for (int c0 = 0; rT && c0 < kx; c0 += 64) {
     for (int i = tid; i < kRouteTok * CPR; i += NT) {
       const int rl = i / CPR, q = i - rl * CPR, tt = t0 + rl, col0 = c0 + q * VEC;
-      Chunk<T> cs, cg, od, os;
-      cs.raw = cg.raw = zero4();
-      if (tt < N) {
-        cs.raw = *(const u32x4*)(Sb + (size_t)rl * kx + col0);
-        cg.raw = *(const u32x4*)(Gb + (size_t)rl * kx + col0);
-      }
+      Chunk<T> od, os;
+      scaled(rl, col0, od, os);
 #pragma unroll
       for (int j = 0; j < VEC; ++j) {
-        const int col = col0 + j, e = col / r;
-        float g = 0.f;
-        if (col < E * r)
-          for (int s = 0; s < kBwdMaxK; ++s)
-            if (es[rl][s] == e) g = gs[rl][s];
-        od.e[j] = from_f<T>(g * to_f(cg.e[j]));
-        os.e[j] = from_f<T>(g * to_f(cs.e[j]));
         tD[q * VEC + j][rl] = od.e[j];
         tS[q * VEC + j][rl] = os.e[j];
       }
@@ -314,7 +325,7 @@ __global__ __launch_bounds__(kRouteThreads) void bwd_route_kernel(
       if (sgd && tt < N) *(u32x4*)(sgd + (size_t)tt * kx + col0) = os.raw;
     }
     __syncthreads();
-    for (int i = tid; rT && i < 64 * TPR; i += NT) {
+    for (int i = tid; i < 64 * TPR; i += NT) {
       const int cl = i / TPR, q = i - cl * TPR;
       Chunk<T> od, os;
 #pragma unroll

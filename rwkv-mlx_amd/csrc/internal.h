@@ -311,6 +311,23 @@ hipError_t launch_bwd_finish_expert(int dtype, const float* part_a, const float*
 hipError_t launch_bwd_finish(int dtype, const float* part_o, int ks_o, const void* o, int E, int C, int r, int kx,
                              int ep, void* dA, void* dwg, const float* part_b, int ks_b, void* dB, hipStream_t s);
 
+// fp32 layers of few tokens (bwd_f32_direct, bwd_f32.hip).  First: S = x·A_all,
+// G = dO·B_allᵀ (N x kx, zero past E·r) and the selection counts.  Last: dx, dA,
+// dB and dW_gate from DSd, SGd (N x kx) and dℓ (N x ep); null outputs are
+// skipped.
+bool bwd_f32_direct(int dtype, int N, int C, int E, int r);
+hipError_t launch_bwd_f32_first(const float* x, const float* dO, const float* A, const float* B, const int* inds, int N,
+                                int C, int E, int k, int r, int kx, float* S, float* G, int* cnt, hipStream_t s);
+hipError_t launch_bwd_f32_last(const float* x, const float* dO, const float* A, const float* wg, const float* dsd,
+                               const float* sgd, const float* dl, int N, int C, int E, int r, int kx, int ep, float* dx,
+                               float* dA, float* dB, float* dwg, hipStream_t s);
+// The gradient of orthogonal_loss in two launches on fp32 MFMA, where that is
+// ahead of the GEMM tiles (`gram`: ortho_gram_bytes of scratch).
+bool ortho_backward_direct(int dtype, int E, int C, int r);
+size_t ortho_gram_bytes(int E, int r);
+hipError_t launch_ortho_backward(int dtype, const void* A, int E, int C, int r, const float* d_ortho, float* gram,
+                                 void* dA, hipStream_t s);
+
 // LoRA helpers, grouped LoRA, combine, orthogonality loss.
 int lora_kx(int E, int r);
 // A_all and B_all in one launch.
