@@ -21,8 +21,8 @@
 //      phases 1b-4 (issued after the tile's loads: a wave's loads complete in
 //      order, so the tile does not wait behind them);
 //      1b. optional: xk = x + (shift(x) - x) * x_k for the tile's rows;
-//   2. the TT·E·(C/64) chunk dot products, as 2x2 (token, expert) micro-tiles
-//      (2x4 for bf16); consecutive lanes take consecutive expert groups, then
+//   2. the TT·E·(C/64) chunk dot products, on v_mfma_f32_4x4x1 for bf16 with
+//      several tiles a CU, else as 2x2 (token, expert) micro-tiles (2x4 for bf16); consecutive lanes take consecutive expert groups, then
 //      token pairs, so a wave's LDS reads hit distinct banks;
 //   3. chunks are summed per (token, expert) and rounded to fp32 (for E <= 32
 //      by the lane that routes that pair in phase 4);
@@ -101,17 +101,29 @@ struct RouterSmem {
 template <typename T, typename WT>
 using logit_acc_t = typename std::conditional<sizeof(T) == 2 && sizeof(WT) == 2, float, double>::type;
 
+// The plan of chunk_mfma (`mf`): the chunk sums lie as Q rows of TT·E (+ 4, so
+// that the chunks of a wave's stores lie in different banks), over the two
+// rows that only the shift mix reads.
+__host__ __device__ inline int part_stride(int TT, int E) { return TT * E + 4; }
+
 // `ln`: ln2's weight and bias (C elements each) after the rest, for the
 // kernels that normalize their tile.
 template <typename T, typename WT>
-__host__ __device__ RouterSmem router_smem(int TT, int C, int E, bool w_ok, bool ln = false) {
+__host__ __device__ RouterSmem router_smem(int TT, int C, int E, bool w_ok, bool ln = false, bool mf = false) {
   RouterSmem m;
   const int XS = C + 16 / (int)sizeof(T);
   const int WS = C + 16 / (int)sizeof(WT);  // W_gate rows in LDS, 16 B padding
-  const size_t part = (size_t)TT * E * (C / 64) * sizeof(logit_acc_t<T, WT>);
-  m.part = 0;
-  m.xs = (part + 15) / 16 * 16;
-  m.ws = m.xs + (size_t)(TT + 2) * XS * sizeof(T);  // tile rows, the row before the tile, x_k
+  const size_t row = (size_t)XS * sizeof(T), acc = sizeof(logit_acc_t<T, WT>);
+  if (mf) {
+    const size_t part = (size_t)part_stride(TT, E) * (C / 64) * acc;
+    m.xs = 0;
+    m.part = TT * row;
+    m.ws = m.part + (part > 2 * row ? (part + 15) / 16 * 16 : 2 * row);
+  } else {
+    m.part = 0;
+    m.xs = ((size_t)TT * E * (C / 64) * acc + 15) / 16 * 16;
+    m.ws = m.xs + (TT + 2) * row;  // tile rows, the row before the tile, x_k
+  }
   // lg, gd, prob (TT*E floats each), zt (16 floats), selected-expert masks (16
   // uint64; zt and the masks are read for 16 rows, zeros past the tile)
   const size_t tail = (size_t)TT * E * 3 * sizeof(float) + 16 * sizeof(float) + 8 + 16 * 8;
@@ -493,14 +505,16 @@ struct RouterLn {
 // fragments per K-step (2: fp32 adapters as fp16 pairs, T = f16 only); KT:
 // the decode front (decode_router_groups(N) workgroups of the wave-per-token
 // router, then the decode key and adapter tiles); LN: x is the residual
-// stream and the tile's rows are LN(x) (not with KT).
-template <typename T, typename WT, int EB, bool WU, int FPK, bool KT, bool LN = false>
-__global__ __launch_bounds__(kRouterThreads) __attribute__((amdgpu_waves_per_eu(KT ? 4 : (std::is_same<T, f16>::value && std::is_same<WT, f16>::value && !WU && EB <= 32 ? 8 : 1)))) void router_kernel(
+// stream and the tile's rows are LN(x) (not with KT); MF: the chunk products
+// on MFMAs (bf16, several tiles a CU).
+template <typename T, typename WT, int EB, bool WU, int FPK, bool KT, bool LN = false, bool MF = false>
+__global__ __launch_bounds__(kRouterThreads) __attribute__((amdgpu_waves_per_eu(KT ? 4 : (std::is_same<T, f16>::value && std::is_same<WT, f16>::value && !WU && EB <= 32 ? 8 : (MF && EB <= 32 ? 6 : 1))))) void router_kernel(
     const T* __restrict__ x, const WT* __restrict__ wg, const float* __restrict__ bias, const T* __restrict__ xprev,
     const T* __restrict__ mu, const T* __restrict__ at, int N, int T_, int C, int E, int k, int r, int TT,
     float* logits, int* inds, T* gates, T* gate_dense, T* xk, T* u_arg, double* part_f64, int* part_cnt,
     int* loss_claim, int opts, int nbr, DecodeKey<T> dk, RouterLn<T> ln) {
   static_assert(!(KT && LN), "the decode front reads LN(x) written by layer_norm_kernel");
+  static_assert(!MF || (std::is_same<T, bf16>::value && std::is_same<T, WT>::value && !WU && !KT), "bf16, no adapters");
   static_assert(FPK == 1 || (FPK == 2 && std::is_same<T, f16>::value), "fp16 pairs need an fp16 layer");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   // the argument lines at offsets 0x00 (x), 0x40 (k), 0x80 (part_f64), 0xc0 (dk.kx)
@@ -520,11 +534,12 @@ __global__ __launch_bounds__(kRouterThreads) __attribute__((amdgpu_waves_per_eu(
   constexpr int VEC = 16 / sizeof(T);
   constexpr bool WSAME = std::is_same<T, WT>::value;
   // opts bit 0: W_gate staged in LDS; bit 1: U without the gates (u)
-  const RouterSmem sm = router_smem<T, WT>(TT, C, E, (opts & 1) != 0, LN);
+  const RouterSmem sm = router_smem<T, WT>(TT, C, E, (opts & 1) != 0, LN, MF);
   T* const u = WU ? u_arg : nullptr;  // the instance without U drops its registers
   const int Q = C / 64, XS = xs_stride<T>(C), WS = C + 16 / (int)sizeof(WT);
   typedef logit_acc_t<T, WT> acc_t;
-  acc_t* part = (acc_t*)smem;                      // TT*E*Q chunk dot products
+  acc_t* part = (acc_t*)(smem + sm.part);          // the chunk dot products
+  const int PS = part_stride(TT, E);               // (MF: chunk q of pair p at q*PS + p, else at p*Q + q)
   T* xs = (T*)(smem + sm.xs);                      // TT*XS
   float* lg = (float*)(smem + sm.lg);              // TT*E logits
   float* gd = lg + TT * E;                         // TT*E dense gates (0 where not routed)
@@ -534,6 +549,7 @@ __global__ __launch_bounds__(kRouterThreads) __attribute__((amdgpu_waves_per_eu(
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int t0 = blockIdx.x * TT;
+  const int nt = min(TT, N - t0);
   // the loss reduction of this forward is claimed later by the first key GEMM
   // workgroup to finish (kernels on one stream run in order)
   // (and the dispatch ticket beside it, claim[1], for a dispatch job in the
@@ -542,7 +558,6 @@ __global__ __launch_bounds__(kRouterThreads) __attribute__((amdgpu_waves_per_eu(
     loss_claim[0] = 0;
     loss_claim[1] = 0;
   }
-  const int nt = min(TT, N - t0);
 
   // adapter down-projection operands: this wave's 16 columns of A_all
   using UM = Mma16<T>;
@@ -571,6 +586,23 @@ __global__ __launch_bounds__(kRouterThreads) __attribute__((amdgpu_waves_per_eu(
   // barrier
   constexpr int UB = UCH / 4;
 
+  // chunk_mfma's tasks, and W_gate in registers where it is not staged: a
+  // lane's expert row of one chunk, whole (8 pieces of 16 bytes: each of its
+  // cache lines is fetched once)
+  constexpr int NP = 64 / VEC;
+  // one or two rows of blocks a task: two where every wave still has a task
+  const bool mf2 = MF && (E + 3) / 4 * (((TT + 7) / 8 * Q + 15) / 16) >= kRouterThreads / 64;
+  const int mfTB = (TT + (mf2 ? 7 : 3)) / (mf2 ? 8 : 4), mf_items = mfTB * Q, mf_ng = (mf_items + 15) / 16;
+  const int mf_tasks = (E + 3) / 4 * mf_ng;
+  u32x4 wpre[NP];
+  auto w_prefetch = [&](int task) {
+    const int tk = min(task, mf_tasks - 1), eb = tk / mf_ng;
+    const int jc = min((tk - eb * mf_ng) * 16 + (lane >> 2), mf_items - 1);
+    const T* wr = (const T*)wg + (size_t)min(eb * 4 + (lane & 3), E - 1) * C + jc / mfTB * 64;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) wpre[i] = *(const u32x4*)(wr + i * VEC);
+  };
+
   // 1. x tile, the row before it and x_k (both for xk), and W_gate -> LDS,
   //    up to LB 16-byte loads per thread in flight before any is stored.
   //    The LDS rows are consecutive (tile rows, prev, x_k, then W_gate), so
@@ -596,6 +628,7 @@ __global__ __launch_bounds__(kRouterThreads) __attribute__((amdgpu_waves_per_eu(
     const T* prev_src = t0 % T_ != 0 ? x + (size_t)(t0 - 1) * C : (xprev ? xprev + (size_t)(t0 / T_) * C : x);
     const T* mu_src = mu ? mu : x;
     constexpr int LB = 8;
+    T* const wrows = MF ? (T*)(smem + sm.ws) - (size_t)(TT + 2) * XS : xs;  // where W_gate's rows count from
     int R = tid / cpr, cc = tid % cpr;
     for (int b0 = 0; b0 < nrows * cpr; b0 += LB * kRouterThreads) {
       u32x4 v[LB];
@@ -622,7 +655,7 @@ __global__ __launch_bounds__(kRouterThreads) __attribute__((amdgpu_waves_per_eu(
       }
 #pragma unroll
       for (int j = 0; j < LB; ++j)
-        if (rr[j] < nrows) *(u32x4*)(xs + (size_t)rr[j] * XS + cs[j]) = v[j];
+        if (rr[j] < nrows) *(u32x4*)((rr[j] < TT + 2 ? xs : wrows) + (size_t)rr[j] * XS + cs[j]) = v[j];
     }
   }
   // an fp32 W_gate beside a 16-bit x: its rows go to LDS in a loop of their
@@ -652,7 +685,9 @@ __global__ __launch_bounds__(kRouterThreads) __attribute__((amdgpu_waves_per_eu(
     for (int i = tid + kRouterThreads; i < 2 * cpr; i += kRouterThreads)  // rows of more than 256 chunks
       *(u32x4*)(lnl + (size_t)i * VEC) = *(const u32x4*)(i < cpr ? ln.w + i * VEC : ln.b + (i - cpr) * VEC);
   }
-  asm volatile("" ::: "memory");  // the tile's loads and LDS stores stay ahead of the prefetch
+  asm volatile("" ::: "memory");  // the tile's loads and LDS stores stay ahead of the prefetches
+  if constexpr (MF)
+    if (!sm.w_in_lds) w_prefetch(wave);
   if (u) u_load(0, 0, UB);
   lds_barrier();
   if constexpr (LN) {
@@ -863,23 +898,96 @@ __global__ __launch_bounds__(kRouterThreads) __attribute__((amdgpu_waves_per_eu(
       for (int m = 0; m < MT; ++m) part[((size_t)min(tb * MT + m, TT - 1) * E + e) * Q + q] = a[m];
     }
   };
-  if (sm.w_in_lds) chunk_dots((const WT*)(smem + sm.ws), WS);
-  else if constexpr (std::is_same<T, f16>::value && WSAME && !WU && !KT) chunk_cols();  // (the decode front stages W_gate)
-  else chunk_dots(wg, C);
+  // bf16, several tiles a CU: the same chains on v_mfma_f32_4x4x1, whose K is one
+  // term, so that an instruction is one single-rounding FMA for each of 16
+  // blocks of 4 tokens x 4 experts.  A lane takes token (expert) lane % 4 of
+  // block lane / 4; a block is one chunk, and a wave's task is 16 blocks x RT
+  // token rows of blocks for one group of 4 experts.  It runs at twice the
+  // VALU's FMA rate, and an operand's conversion feeds 4 (4·RT) FMAs of its
+  // lane's block.
+  auto chunk_mfma = [&](auto rt, auto staged) {
+    constexpr int RT = decltype(rt)::value;
+    constexpr bool WL = decltype(staged)::value;
+    const int l4 = lane & 3;
+    for (int task = wave, it = 0; it * (kRouterThreads / 64) < mf_tasks; task += kRouterThreads / 64, ++it) {
+      const int eb = task / mf_ng, j = (task - eb * mf_ng) * 16 + (lane >> 2);
+      const int jc = min(j, mf_items - 1), q = jc / mfTB, tb = jc - q * mfTB, e = eb * 4 + l4;
+      f32x4 acc[RT];
+#pragma unroll
+      for (int r = 0; r < RT; ++r) acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (task < mf_tasks) {  // (the whole wave)
+        if (!WL && it > 0) w_prefetch(task);
+        const T* xr[RT];
+        const T* wr = (const T*)(smem + sm.ws) + (size_t)min(e, E - 1) * WS + q * 64;
+        Chunk<T> wl[2];
+        if constexpr (WL) wl[0].raw = *(const u32x4*)wr;
+        Chunk<T> cx[2][RT];
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+          xr[r] = xs + (size_t)min((tb * RT + r) * 4 + l4, TT - 1) * XS + q * 64;
+          cx[0][r].raw = *(const u32x4*)xr[r];
+        }
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+          if (i + 1 < NP) {
+#pragma unroll
+            for (int r = 0; r < RT; ++r) cx[(i + 1) & 1][r].raw = *(const u32x4*)(xr[r] + (i + 1) * VEC);
+          }
+          if (WL && i + 1 < NP) wl[(i + 1) & 1].raw = *(const u32x4*)(wr + (i + 1) * VEC);
+          Chunk<T> w;
+          w.raw = WL ? wl[i & 1].raw : wpre[i];
+#pragma unroll
+          for (int v = 0; v < VEC; ++v) {
+            const float fw = to_f(w.e[v]);
+#pragma unroll
+            for (int r = 0; r < RT; ++r)
+              acc[r] = __builtin_amdgcn_mfma_f32_4x4x1f32(to_f(cx[i & 1][r].e[v]), fw, acc[r], 0, 0, 0);
+          }
+        }
+      }
+      if (it == 0) lds_barrier();  // every wave is past the mix: its two rows become the chunk sums'
+      if (task < mf_tasks && j < mf_items && e < E) {
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const int tl = (tb * RT + r) * 4 + v;
+            if (tl < TT) part[q * PS + tl * E + e] = acc[r][v];
+          }
+      }
+    }
+  };
+  if constexpr (MF) {
+    typedef std::integral_constant<int, 1> one;
+    typedef std::integral_constant<int, 2> two;
+    if (sm.w_in_lds) {
+      if (mf2) chunk_mfma(two{}, std::true_type{});
+      else chunk_mfma(one{}, std::true_type{});
+    } else {
+      if (mf2) chunk_mfma(two{}, std::false_type{});
+      else chunk_mfma(one{}, std::false_type{});
+    }
+  } else {
+    if (sm.w_in_lds) chunk_dots((const WT*)(smem + sm.ws), WS);
+    else if constexpr (std::is_same<T, f16>::value && WSAME && !WU && !KT) chunk_cols();  // (the decode front stages W_gate)
+    else chunk_dots(wg, C);
+  }
   lds_barrier();
 
   // 3. chunk sums in ascending order, one rounding to fp32 (+ bias).  With
   //    E <= 32 the lane that routes (token, expert) in phase 4 computes it
   //    there; otherwise here, into lg.
   auto logit_of = [&](int tl, int e) -> float {
-    const acc_t* pp = part + (size_t)(tl * E + e) * Q;
+    const acc_t* pp = part + (MF ? tl * E + e : (tl * E + e) * Q);
+    const int ps = MF ? PS : 1;
+    constexpr int QB = MF ? 8 : 4;
     double s = 0.0;
-    for (int q0 = 0; q0 < Q; q0 += 4) {  // loads of 4 chunks in flight, added in ascending q
-      double v[4];
+    for (int q0 = 0; q0 < Q; q0 += QB) {  // loads of QB chunks in flight, added in ascending q
+      double v[QB];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = (double)pp[min(q0 + i, Q - 1)];
+      for (int i = 0; i < QB; ++i) v[i] = (double)pp[min(q0 + i, Q - 1) * ps];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < QB; ++i)
         if (q0 + i < Q) s += v[i];
     }
     float l = (float)s;
@@ -1159,11 +1267,11 @@ __global__ __launch_bounds__(kRouterThreads) __attribute__((amdgpu_waves_per_eu(
 // 8-token tiles the overlapping load / FMA / routing phases of several
 // workgroups are worth more than reading W_gate from LDS instead of L2.
 template <typename T, typename WT>
-int router_w_in_lds_ok(int nb, int TT, int C, int E, bool with_u, bool ln) {
+int router_w_in_lds_ok(int nb, int TT, int C, int E, bool with_u, bool ln, bool mf) {
   if (with_u) return 1;  // the adapter instance's registers allow one workgroup per CU
   const int cus = num_cus(), want = (nb + cus - 1) / cus;
   auto occ = [&](bool w) {
-    const int o = kLdsBytes / (int)router_smem<T, WT>(TT, C, E, w, ln).total;
+    const int o = kLdsBytes / (int)router_smem<T, WT>(TT, C, E, w, ln, mf).total;
     return o < want ? o : want;
   };
   return occ(true) >= occ(false);
@@ -1201,9 +1309,16 @@ hipError_t launch_router(int dtype, bool gate32, int fpk, const void* x, const v
   auto go = [&](auto tag_t, auto tag_w) -> hipError_t {
     typedef decltype(tag_t) T;
     typedef decltype(tag_w) WT;
-    const int w_ok = front ? 1 : router_w_in_lds_ok<T, WT>(nb, TT, C, E, u != nullptr, ln_w != nullptr);
+    // The chunk products on MFMAs: where a CU has several tiles, their FMAs
+    // and operand conversions bound the kernel (bf16 16384 x 2048, E=16: 102 ->
+    // 67 us, and 3 workgroups a CU instead of 2).  A CU's only tile waits for
+    // one chain's latency, where the VALU's is the shorter (127 tiles of 16 x
+    // 1024, E=8: 16.6 against 17.3 us; 50 of 4 x 2048, E=16: 15.0 / 15.8), and
+    // fp16 converts inside the VALU's FMA (8192 x 1024, E=32: 34 / 37).
+    const bool mf = std::is_same<T, bf16>::value && std::is_same<T, WT>::value && !front && !u && nb > num_cus();
+    const int w_ok = front ? 1 : router_w_in_lds_ok<T, WT>(nb, TT, C, E, u != nullptr, ln_w != nullptr, mf);
     const int opts = w_ok | (u_raw ? 2 : 0);
-    size_t smem = router_smem<T, WT>(TT, C, E, w_ok != 0, ln_w != nullptr).total;
+    size_t smem = router_smem<T, WT>(TT, C, E, w_ok != 0, ln_w != nullptr, mf).total;
     DecodeKey<T> dk{nullptr, nullptr, 0, nullptr, nullptr, 0, 0, nullptr};
     const RouterLn<T> lnp{(const T*)ln_w, (const T*)ln_b, (T*)xn};
     int grid = nb;
@@ -1246,6 +1361,18 @@ hipError_t launch_router(int dtype, bool gate32, int fpk, const void* x, const v
       if (E <= 8) return RWKV_ROUTER(8, true, 1);
       if (E <= 16) return RWKV_ROUTER(16, true, 1);
       return hipErrorInvalidValue;  // E * r <= 128 with r >= 8
+    }
+    if constexpr (std::is_same<T, bf16>::value && std::is_same<T, WT>::value) {
+      if (mf) {
+#define RWKV_ROUTER_MF(EB)                                                       \
+  (ln_w ? launch(router_kernel<T, WT, EB, false, 1, false, true, true>)          \
+        : launch(router_kernel<T, WT, EB, false, 1, false, false, true>))
+        if (E <= 8) return RWKV_ROUTER_MF(8);
+        if (E <= 16) return RWKV_ROUTER_MF(16);
+        if (E <= 32) return RWKV_ROUTER_MF(32);
+        return RWKV_ROUTER_MF(64);
+#undef RWKV_ROUTER_MF
+      }
     }
     if (E <= 8) return RWKV_ROUTER(8, false, 1);
     if (E <= 16) return RWKV_ROUTER(16, false, 1);
