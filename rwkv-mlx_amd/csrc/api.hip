@@ -537,7 +537,9 @@ BwdLayout bwd_layout(const Dims& d) {
   L.dx32 = bwd_f32_direct(d.dtype, d.N, d.C, d.E, d.r);
   L.ox = ortho_backward_direct(d.dtype, d.E, d.C, d.r);
   const size_t sg = L.fx ? 0 : 1;     // S and G in memory
-  const size_t dense = L.px || L.dx32 ? 0 : 1;  // the dense token-contracted products
+  // the dense token-contracted products; an fp32 layer's workspace holds them
+  // whichever form its products take (bwd_f32_direct)
+  const size_t dense = L.px ? 0 : 1;
   const size_t px = L.px ? 1 : 0;
   L.at = take(kx * C * s);
   L.a_t = take(C * kx * s);
