@@ -214,29 +214,29 @@ hipError_t launch_experts_mix(int dtype, const void* x, const void* xprev, const
 
 // Full-expert backward (experts_bwd.hip); rows j in perm order (nk = N·k).
 // dO rows gathered (dog, nk x C) and each row's gate gr (fp32, the forward's
-// rounding) recomputed from logits and inds.
+// rounding) recomputed from logits and inds; and the packed token ranges of
+// the weight-gradient products (koff, E + 1 ints): expert e's rows take
+// columns [koff[e], koff[e+1]), its count rounded up to 128 (128 when it has
+// none); exb_seg_cols(nk, E) bounds koff[E] (a multiple of 128).
 hipError_t launch_exb_gather(int dtype, const void* dO, const int* perm, const float* logits, const int* inds,
-                             int nk, int C, int E, int k, void* dog, float* gr, hipStream_t s);
-// From p (nk x F, the key product before relu²) and u = dO·W_val (nk x F):
-// dw[j] = <relu(p)², u> (fp32) and dp = g·u·2·relu(p), written over u's rows
-// when dp == U (each element is read before it is written).
-hipError_t launch_exb_hidden(int dtype, const void* P, const void* U, const float* gr, int nk, int F, void* dp,
-                             float* dw, hipStream_t s);
-// The packed token ranges of the weight-gradient products (koff, E + 1
-// ints): expert e's rows take columns [koff[e], koff[e+1]), its count
-// rounded up to 128 (128 when it has none); exb_seg_cols(nk, E) bounds
-// koff[E] (a multiple of 128).
-hipError_t launch_exb_koff(const int* off, int E, int* koff, hipStream_t s);
+                             const int* off, int nk, int C, int E, int k, void* dog, float* gr, int* koff,
+                             hipStream_t s);
 int exb_seg_cols(int nk, int E);
-// dst (W x ld) with range e (columns [koff[e], koff[e+1])) the transpose of
-// src rows [off[e], off[e+1]) (nk x W), zero past the count.  mode 0 copies,
-// 1 writes round(relu(v)²), 2 writes round(v · gr[row]).  W % 64, ld % 128.
-hipError_t launch_exb_seg_transpose(int dtype, int mode, const void* src, int W, const int* off, const int* koff,
-                                    int E, int ld, const float* gr, void* dst, hipStream_t s);
-// Router cotangents dl (N x E, fp32) from the slot cotangents dw (perm
-// order) and the loss cotangents (dloss: [d_aux, d_z] or null).
-hipError_t launch_exb_route(const float* logits, const int* inds, const int* inv, const float* dw, const int* off,
-                            const float* dloss, int N, int E, int k, float* dl, hipStream_t s);
+// From p (nk x F, the key product before relu²) and u = dO·W_val (nk x F):
+// dp = g·u·2·relu(p) over u, its packed transpose dpT and that of h =
+// round(relu(p)²), hT (F x ld each, zero past an expert's rows; null: not
+// written), and dwp (F/64 x nk): the parts of dw[j] = <h_j, u_j> per 64 columns.
+hipError_t launch_exb_hidden(int dtype, const void* P, const float* gr, const int* off, const int* koff, int E, int nk,
+                             int F, int ld, void* U, void* dpT, void* hT, float* dwp, hipStream_t s);
+// Packed transposes dst0 of src0 and dst1 of round(src1 · gr[row]) (W x ld
+// each; null: not written).  W % 64, ld % 128.
+hipError_t launch_exb_seg_transpose(int dtype, const void* src0, const void* src1, int W, const int* off,
+                                    const int* koff, int E, int ld, const float* gr, void* dst0, void* dst1,
+                                    hipStream_t s);
+// Router cotangents dl (N x E, fp32) from np parts of the slot cotangents (dwp,
+// np x N·k, perm order) and the loss cotangents (dloss: [d_aux, d_z] or null).
+hipError_t launch_exb_route(const float* logits, const int* inds, const int* inv, const float* dwp, int np,
+                            const int* off, const float* dloss, int N, int E, int k, float* dl, hipStream_t s);
 // The standalone router's dl (N x E, fp32): the gates' cotangents d_gates
 // (N x k, dtype, assignment order t·k + s; may be null) through the
 // selected-logit softmax, plus the loss cotangents; counts from off.
