@@ -538,7 +538,8 @@ BwdLayout bwd_layout(const Dims& d) {
   L.ox = ortho_backward_direct(d.dtype, d.E, d.C, d.r);
   const size_t sg = L.fx ? 0 : 1;     // S and G in memory
   // the dense token-contracted products; an fp32 layer's workspace holds them
-  // whichever form its products take (bwd_f32_direct)
+  // whichever form its products take, so that it does not shrink where more
+  // tokens leave the direct form (bwd_f32_direct)
   const size_t dense = L.px ? 0 : 1;
   const size_t px = L.px ? 1 : 0;
   L.at = take(kx * C * s);
@@ -556,12 +557,13 @@ BwdLayout bwd_layout(const Dims& d) {
   L.sgdT = take(dense * kx * np * s);
   L.o = take(C * (kx + ep) * s);
   L.xp = bwd_expert_plan(d.N, d.C, d.E, d.k);
-  L.sgd = take((L.px || L.dx32 ? 1 : 0) * N * kx * s);
+  // (the direct form's SGd lies where the dense products keep its transpose)
+  L.sgd = L.dx32 ? L.sgdT : take(px * N * kx * s);
   L.emask = take(px * N * sizeof(unsigned long long));
   L.pa = take(px * (size_t)d.E * L.xp.R * C * d.r * sizeof(float));
   L.pb = take(px * (size_t)d.E * L.xp.R * C * d.r * sizeof(float));
   L.pw = take(px * (size_t)L.xp.RW * d.E * C * sizeof(float));
-  L.gram = take(std::max(L.ox ? ortho_gram_bytes(d.E, d.r) : 0, kx * kx * s));
+  L.gram = take(kx * kx * s);
   size_t sk = gemm_nt_partial_bytes(d.dtype, d.N, d.kx, d.C, GEMM_HINT_NO_SPLIT);
   sk = std::max(sk, gemm_nt_partial_bytes(d.dtype, d.C, d.kx + L.ep, L.np));
   sk = std::max(sk, gemm_nt_partial_bytes(d.dtype, d.N, d.C, d.kx + L.ep));
@@ -571,6 +573,10 @@ BwdLayout bwd_layout(const Dims& d) {
   // dB's partials live beside O's until bwd_finish reduces both
   L.splitk_b = take(dense * gemm_nt_partial_bytes(d.dtype, d.E * d.r, d.C, L.np, GEMM_HINT_SPLIT64));
   L.total = off;
+  if (L.ox) {  // the direct orthogonality gradient's fp32 Gram matrix is all that it keeps
+    L.gram = 0;
+    L.total = std::max(L.total, (ortho_gram_bytes(d.E, d.r) + 255) / 256 * 256);
+  }
   return L;
 }
 

@@ -384,6 +384,16 @@ def test_backward_workspace_sizes(L):
     assert L.lib().rwkvmoe_backward_workspace_bytes(ctypes.byref(desc(L)), None) == -4
 
 
+@pytest.mark.parametrize("kw,tokens", [(dict(lora_rank=24), 5461),
+                                       (dict(n_experts=5, lora_rank=16, d_model=64, d_ffn=64), 157286)])
+def test_fp32_backward_workspace_serves_both_forms(L, kw, tokens):
+    """`tokens` is the largest batch whose fp32 products run on the operands as
+    stored: a workspace sized one token above serves it too."""
+    size = lambda n: bwd_ws(L, desc(L, dtype="f32", batch=1, seq_len=n, **kw))
+    (s0, direct), (s1, dense) = size(tokens), size(tokens + 1)
+    assert s0 == 0 and s1 == 0 and direct <= dense
+
+
 def test_backward_argument_errors(L):
     d = desc(L)
     assert bwd_status(L, None, fake_grads(L), ws_bytes=1 << 30) == -1
