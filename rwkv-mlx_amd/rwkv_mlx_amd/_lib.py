@@ -419,7 +419,10 @@ class KernelTimer:
 
 
 def current_stream(device) -> int:
-    """The hipStream_t of torch's current stream on `device` (without the
-    Stream object that torch.cuda.current_stream makes, 2.5 us a call)."""
+    """The hipStream_t of torch's current stream on `device` (anything that
+    torch.cuda.current_stream takes; for a CUDA torch.device without the Stream
+    object that it makes, 2.5 us a call)."""
+    if not isinstance(device, torch.device) or device.type != "cuda":
+        return torch.cuda.current_stream(device).cuda_stream  # (raises for what is no CUDA device)
     index = device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)

@@ -143,3 +143,18 @@ def test_empty_input():
     inds, w, aux2, z2 = m.router(x)
     assert inds.shape == (0, 7, 2) and math.isnan(float(aux2))
     assert m.base(x).shape == (0, 7, 128)
+
+
+def test_stream_handle_of_any_device_form():
+    """The launches' stream lookup takes what torch.cuda.current_stream takes,
+    and refuses what it refuses."""
+    import torch
+    from rwkv_mlx_amd import _lib
+    side = torch.cuda.Stream()
+    for stream in (torch.cuda.current_stream(), side):
+        with torch.cuda.stream(stream):
+            for dev in (torch.device("cuda", 0), torch.device("cuda"), "cuda:0", "cuda", 0, None):
+                assert _lib.current_stream(dev) == stream.cuda_stream, dev
+    for dev in (torch.device("cpu"), "cpu"):
+        with pytest.raises(ValueError):
+            _lib.current_stream(dev)
