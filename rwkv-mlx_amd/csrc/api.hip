@@ -832,9 +832,12 @@ int experts_forward_impl(const rwkvmoe_desc* desc, const rwkvmoe_tensors* t, voi
   return RWKVMOE_OK;
 }
 
-// Workspace of rwkvmoe_experts_backward.  np: tokens padded to 128, the
-// length of each expert's segment in the token-major (transposed) operands of
-// the weight-gradient products.
+// Workspace of rwkvmoe_experts_backward.  The weight-gradient products read
+// token-major (transposed) operands of ncol columns.  Those of the hidden
+// columns (dpᵀ, hᵀ) come from the hidden pass and have regions of their own;
+// xkᵀ and (g·dO)ᵀ come after dk's last reader and lie over P, U, W_eᵀ and dk,
+// which nothing reads any more.  The parts of dw lie in dk, which is written
+// after the routing kernel has added them.
 struct ExpBwdLayout {
   size_t dcounts, perm, inv, offsets, koff, xkg, P, dog, gr, U, dw, wT, dk, dl, cpart, dpT, hT, xT, doT, total;
   int ncol;  // bound on the packed token columns of the transposed operands
@@ -856,19 +859,23 @@ ExpBwdLayout exp_bwd_layout(const Dims& d) {
   L.offsets = take((E + 1) * sizeof(int));
   L.koff = take((E + 1) * sizeof(int));
   L.xkg = take(nk * C * s);
-  L.P = take(nk * F * s);
   L.dog = take(nk * C * s);
   L.gr = take(nk * sizeof(float));
-  L.U = take(nk * F * s);  // u, then dp in place
-  L.dw = take(F / 64 * nk * sizeof(float));
-  L.wT = take(E * F * C * s);  // W_val,eᵀ, then W_key,eᵀ
-  L.dk = take(nk * C * s);
   L.dl = take((size_t)d.N * E * sizeof(float));
   L.cpart = take(E * (size_t)exb_col_chunks(d.N, d.C, d.E) * C * sizeof(float));
   L.dpT = take(F * (size_t)L.ncol * s);
   L.hT = take(F * (size_t)L.ncol * s);
+  const size_t shared = off;
+  L.P = take(nk * F * s);
+  L.U = take(nk * F * s);      // u, then dp in place
+  L.wT = take(E * F * C * s);  // W_val,eᵀ, then W_key,eᵀ
+  L.dk = take(std::max(nk * C * s, F / 64 * nk * sizeof(float)));
+  L.dw = L.dk;
+  const size_t end = off;
+  off = shared;
   L.xT = take(C * (size_t)L.ncol * s);   // xkᵀ
   L.doT = take(C * (size_t)L.ncol * s);  // (g·dO)ᵀ
+  off = std::max(off, end);
   L.total = off;
   return L;
 }
@@ -922,6 +929,9 @@ int experts_backward_impl(const rwkvmoe_desc* desc, const rwkvmoe_experts_grads*
   const int ld = L.ncol;
   HIPTRY(launch_exb_hidden(dt, w + L.P, gr, off, koff, E, nk, F, ld, w + L.U, g->d_w_key ? w + L.dpT : nullptr,
                            g->d_w_value ? w + L.hT : nullptr, dw, s));
+  // router cotangents (from dw, whose region dk takes next)
+  if (g->d_x || g->d_x_prev || g->d_w_gate)
+    HIPTRY(launch_exb_route(g->logits, g->inds, inv, dw, F / 64, off, g->d_losses, N, E, k, dl, s));
   // dk_j = dp_j · W_key,e
   const bool need_dk = g->d_x || g->d_x_prev || g->d_x_k;
   if (need_dk) {
@@ -929,9 +939,6 @@ int experts_backward_impl(const rwkvmoe_desc* desc, const rwkvmoe_experts_grads*
     HIPTRY(launch_grouped_gemm(dt, false, w + L.U, F, w + L.wT, F, (long long)C * F, F, nk, C, off, E, w + L.dk, C,
                                "experts_bwd_dk", s));
   }
-  // router cotangents
-  if (g->d_x || g->d_x_prev || g->d_w_gate)
-    HIPTRY(launch_exb_route(g->logits, g->inds, inv, dw, F / 64, off, g->d_losses, N, E, k, dl, s));
   if (g->d_x || g->d_x_prev)
     HIPTRY(launch_exb_dx(dt, w + L.dk, inv, g->inds, g->x_k, dl, g->w_gate, N, d.T, C, E, k, g->d_x, g->d_x_prev, s));
   if (g->d_x_k)

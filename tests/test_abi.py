@@ -480,6 +480,20 @@ def test_experts_backward_validation(L):
     assert st(grads(), dd=dg) == -3
 
 
+@pytest.mark.parametrize("kw", [dict(), dict(dtype="f32"), dict(d_model=1024, d_ffn=3584),
+                                dict(n_experts=16, top_k=4, d_model=512, d_ffn=1792)])
+def test_experts_backward_workspace_bound(L, kw):
+    """The routed rows' xk, dO and dk, p and u, one expert-weight tensor, and one
+    pair of transposed operands as wide as the larger dimension; beside them
+    the column sums' chunks (at most 256) and the routing's arrays."""
+    d = desc(L, lora_rank=1, **kw)
+    n = ctypes.c_size_t(0)
+    assert L.lib().rwkvmoe_experts_backward_workspace_bytes(ctypes.byref(d), ctypes.byref(n)) == 0
+    N, C, F, E, k, s = d.batch * d.seq_len, d.d_model, d.d_ffn, d.n_experts, d.top_k, 4 if d.dtype == 0 else 2
+    cols = (N * k + 128 * E + 127) // 128 * 128
+    assert n.value <= s * (N * k * (3 * C + 2 * F) + E * F * C + 2 * F * cols) + 4 * 256 * E * C + (1 << 20)
+
+
 def test_gates_f16_flag_is_backward_only(L):
     """RWKVMOE_GATES_F16 (the fine-tune layer's fp32 VJP with fp16 gates):
     accepted by the backward at dtype F32 only; every forward entry point and
