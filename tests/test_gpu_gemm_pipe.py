@@ -109,3 +109,31 @@ def test_row_groups(device, dtype, N, C, F, E, k, hot):
         ref = ref.index_add(0, at, w[at, e:e + 1] * y)
     err = (out - ref).norm().item() / ref.norm().item()
     assert np.isfinite(err) and err <= 5 * UNIT[dtype], err
+
+
+@pytest.mark.parametrize("N,C,F,E,k", [(1, 64, 64, 2, 1), (1, 512, 2048, 4, 1), (9, 64, 64, 64, 8), (64, 512, 2048, 4, 1),
+                                       (200, 768, 3072, 8, 2), (513, 64, 320, 5, 3), (3000, 256, 512, 16, 2),
+                                       (20000, 64, 64, 4, 1)])
+def test_row_groups_reduce_the_losses(device, N, C, F, E, k):
+    """The aux and z losses that the grouped key product reduces, in a workgroup
+    without a tile or in the first to end, against float64 of the same logits;
+    the same bits in every pass."""
+    import torch
+    from rwkv_mlx_amd import MoE_CMix, RWKVConfig
+    torch.manual_seed(N + F)
+    m = MoE_CMix(RWKVConfig(n_embd=C, dim_ffn=F), 0, E, k).to(device=device, dtype=torch.float16).requires_grad_(False)
+    m.expert_key.normal_(0, C ** -0.5)
+    m.expert_val.normal_(0, F ** -0.5)
+    x = torch.randn(1, N, C, device=device).half()
+    ex = {}
+    with torch.no_grad():
+        _, aux, z = m(x, extras=ex)
+        for _ in range(3):
+            _, aux2, z2 = m(x)
+            assert torch.equal(aux, aux2) and torch.equal(z, z2)
+    lg = ex["logits"].double().reshape(N, E)
+    share = torch.zeros(N, E, dtype=torch.float64, device=device).scatter(1, ex["inds"].reshape(N, k).long(), 1.0)
+    ref_aux = E * (share.mean(0) / k * lg.softmax(-1).mean(0)).sum()
+    ref_z = torch.logsumexp(lg, -1).square().mean()
+    assert abs(aux.item() - ref_aux.item()) <= 1e-6 * ref_aux.item()
+    assert abs(z.item() - ref_z.item()) <= 1e-6 * ref_z.item()
