@@ -134,18 +134,26 @@ __global__ __launch_bounds__(512) void pipe_kernel(GemmParams<T> p) {
   const int base = xcd * (total / 8) + min(xcd, total % 8) + (w >> 3);
   const int count = (w >> 3) < run ? (run - (w >> 3) + step - 1) / step : 0;
 
+  constexpr bool JOBS = EPI == EPI_KEYAD;  // only key products are given any
   int ticket = 1;
   // Row groups with fewer tiles than workgroups: the last one, then without a
   // tile, runs the loss reduction beside the others' tiles, and those take no
   // ticket (an atomic each on one address: 0.8 us of the 7.8 that the key
   // product of 64 tokens and 4 experts of 512 x 2048 fp16 took).
-  if (MODE == PIPE_GRP && total < G) ticket = w == G - 1 ? 0 : 2;
+  if constexpr (JOBS && MODE == PIPE_GRP) {
+    if (total < G) ticket = w == G - 1 ? 0 : 2;
+  }
   auto take_ticket = [&]() {
-    if (p.loss.losses != nullptr && tid == 0 && ticket == 1) ticket = atomicAdd(p.loss.claim, 1);
+    if constexpr (!JOBS) return;
+    if constexpr (MODE == PIPE_GRP) {
+      if (ticket != 1) return;
+    }
+    if (p.loss.losses != nullptr && tid == 0) ticket = atomicAdd(p.loss.claim, 1);
   };
   // after the last tile (LDS is free then): the router's loss reduction in
   // the workgroup that took the first ticket, and the dispatch scatter's blocks
   auto run_jobs = [&]() {
+    if constexpr (!JOBS) return;
     if (p.loss.losses != nullptr) {
       __syncthreads();
       int* flag = (int*)lds;
@@ -473,6 +481,7 @@ __global__ __launch_bounds__(512) void pipe_kernel(GemmParams<T> p) {
 
 template <typename T, int BM, int BN, int WGM, int WGN, int L, int EPI, int MODE, bool SPLIT = false>
 hipError_t run_pipe(const GemmParams<T>& p, hipStream_t s) {
+  if (EPI != EPI_KEYAD && (p.loss.losses || p.disp.nblk > 0)) return hipErrorInvalidValue;
   if (p.k1 % 64 || p.k2 % 64 || p.n % BN || (EPI == EPI_KEYAD && p.n_key % BN)) return hipErrorInvalidValue;
   if (MODE == PIPE_GRP && (!p.grp_off || p.grp_n < 1 || p.grp_n > 64)) return hipErrorInvalidValue;
   if (MODE == PIPE_GK && (!p.gk_off || p.gk_n < 1 || p.gk_n > 64)) return hipErrorInvalidValue;
