@@ -803,54 +803,55 @@ TilePlan plan_tiles(int elem, int epi, int m, int n, int n_key, int k_total) {
   return pl;
 }
 
-// ---- 16-bit products: the tile of gemm_pipe.h ----
-// Microseconds of one 64-wide K slice of a tile: `slice` per tile with every CU
-// busy (tiles of which two share a CU: the pair's time over two), `alone` where
-// a CU holds one tile, both measured at K = 8192 with 256 to 4096 tiles (bf16,
-// 16384 x 2048 and 200 to 2031 rows).
-struct PipeTile {
-  int bm, bn, per_cu;
-  double slice, alone;
-};
-constexpr PipeTile kPipeTiles[] = {
-    {256, 256, 1, 1.57, 1.57}, {256, 192, 1, 1.25, 1.25}, {256, 128, 1, 0.87, 0.87}, {128, 192, 1, 0.72, 0.72},
-    {128, 128, 1, 0.53, 0.53}, {128, 128, 2, 0.52, 0.60}, {128, 64, 2, 0.35, 0.30},  {64, 64, 2, 0.22, 0.21},
-};
-
+// ---- 16-bit products: the tile of gemm_pipe.h (kPipeTiles) ----
 struct PipePlan {
   int cfg;    // of kPipeTiles, -1: none fits
   int ks;     // K splits
   double us;  // the model's time
 };
 
-// The tile (and K split) with the least modelled time: rounds of tiles over
-// the CUs times a tile's slices, plus 1 us a round for its epilogue.  With
-// fewer tiles than CUs a slice takes down to 0.7 of its time (L2 and the
-// infinity cache serve fewer CUs).  A split adds the reduction's launch and the
-// fp32 partials' traffic.  A tile never straddles the key / adapter column
-// boundary.  groups: row groups (each may end in a partial tile) or K groups;
-// ld: the operands' row length where it can be long (a tile's rows are
-// addressed with 32 bits).
+// The modelled time of `items` tiles of nk K slices: rounds of tiles over the
+// CUs, each its slices' time and its start and end.  A slice takes its full time
+// in a round with more than 0.88 of the CUs busy, and from there less, down to
+// 0.9 of `alone` (L2 and the infinity cache serve fewer CUs).
+double pipe_us(const PipeTile& t, unsigned items, int nk, int cus) {
+  const unsigned slots = cus * t.per_cu, rounds = items / slots;
+  const int rest = (int)(items - rounds * slots);
+  const double full = nk * t.slice + t.round;
+  double us = (double)rounds * t.per_cu * full;
+  if (rest > cus) us += t.per_cu * full;
+  else if (rest > 0.88 * cus) us += nk * std::max(t.slice, t.alone) + t.round;
+  else if (rest > 0) us += nk * t.alone * (0.9 + 0.1 * (double)rest / cus) + t.round;
+  return us;
+}
+
+// Expected tile rows of m rows in `groups` groups, each of which may end in a
+// partial tile: half a tile row a group, and no fewer than the groups that can
+// hold a row.
+unsigned group_tile_rows(int m, int groups, int bm) {
+  const unsigned g = std::min(groups, m);
+  return std::max(g, (2u * m + (g + 1) * bm) / (2 * bm));
+}
+
+// The tile (and K split) with the least modelled time.  A split adds the
+// reduction's launch, which reads ks partials one after the other, and the fp32
+// partials' way out and back (3.8 TB/s).  A tile never straddles the key / adapter
+// column boundary.  groups: row groups or K groups; ld: the operands' row length
+// where it can be long (a tile's rows are addressed with 32 bits).
 PipePlan plan_pipe(int mode, int m, int n, int n_key, int nkt, int groups = 1, long long ld = 0) {
   const int cus = num_cus();
   PipePlan best{-1, 1, 0.};
-  for (int c = 0; c < (int)(sizeof(kPipeTiles) / sizeof(kPipeTiles[0])); ++c) {
+  for (int c = 0; c < kPipeN; ++c) {
     const PipeTile& t = kPipeTiles[c];
     if (n % t.bn || n_key % t.bn || ld * std::max(t.bm, t.bn) * 2 > 0xFFFFFFF0ll) continue;
-    long long tiles = (long long)((m + t.bm - 1) / t.bm) * (n / t.bn);
-    if (mode == PIPE_GRP) tiles += (long long)(groups / 2) * (n / t.bn);
-    if (mode == PIPE_GK) tiles *= groups;
+    const unsigned rows = mode == PIPE_GRP ? group_tile_rows(m, groups, t.bm) : (unsigned)(m + t.bm - 1) / t.bm;
+    // (below 2^32: an output has fewer than 2^31 elements, of a K group too)
+    const unsigned tiles = rows * (n / t.bn) * (mode == PIPE_GK ? groups : 1);
     const bool split = mode == PIPE_DENSE && (c == 4 || c == 6 || c == 7);
-    for (int ks = 1; ks <= (split ? 16 : 1) && (ks == 1 || nkt / ks >= 4); ++ks) {
-      const long long items = tiles * ks;
-      if (ks > 1 && items > (long long)cus * t.per_cu) break;
-      const long long slots = (long long)cus * t.per_cu, rest = items % slots;
-      const double nk = (double)((nkt + ks - 1) / ks);
-      const double fill = items >= cus ? 1.0 : 0.7 + 0.3 * (double)items / cus;
-      double us = (double)(items / slots) * t.per_cu * (nk * t.slice + 1.0);
-      if (rest > cus) us += t.per_cu * (nk * t.slice + 1.0);
-      else if (rest > 0) us += nk * t.alone * fill + 1.0;
-      if (ks > 1) us += 4.0 + (double)ks * m * n * 8.0 / 3.5e6;
+    const int most = split ? std::min(std::min(16, nkt / 4), (int)((unsigned)(cus * t.per_cu) / tiles)) : 1;
+    for (int ks = 1; ks == 1 || ks <= most; ++ks) {
+      double us = pipe_us(t, tiles * ks, (nkt + ks - 1) / ks, cus);
+      if (ks > 1) us += 2.75 + 0.05 * ks + (double)ks * m * n * 8.0 / 3.8e6;
       if (best.cfg < 0 || us < best.us) best = PipePlan{c, ks, us};
     }
   }
@@ -956,6 +957,15 @@ int num_cus() {
     return n;
   }();
   return v;
+}
+
+int gemm_plan(int mode, int m, int n, int n_key, int k, int groups, int* cfg, int* ks) {
+  if (mode < PIPE_DENSE || mode > PIPE_GK || m < 1 || n < 64 || n % 64 || n_key % 64 || k < 64 || groups < 1 || !cfg || !ks)
+    return -1;
+  const PipePlan p = plan_pipe(mode, m, n, n_key, k / 64, groups);
+  *cfg = p.cfg;
+  *ks = p.ks;
+  return p.cfg < 0 ? -1 : kPipeTiles[p.cfg].per_cu * num_cus();
 }
 
 bool value_plan_mixed_ok(int m, int n, int k_total) {

@@ -81,7 +81,7 @@ __global__ __launch_bounds__(512) void pipe_kernel(GemmParams<T> p) {
   constexpr int DA = BM / 64, DB = BN / 64;  // 1 KB requests of a wave per slice
   static_assert(DA * 64 == BM && DB * 64 == BN, "requests");
   constexpr int UA = BM * RB, UB = BN * RB;
-  constexpr int LDS_BYTES = (L + 1) * UA + L * UB;
+  constexpr int LDS_BYTES = (L + 1) * UA + L * UB;  // (pipe_lds_bytes)
   static_assert(LDS_BYTES <= 163840, "LDS budget");
   constexpr int NT = 512;
   static_assert(256 + loss_scratch_bytes(NT) <= LDS_BYTES, "loss scratch");
@@ -479,8 +479,9 @@ __global__ __launch_bounds__(512) void pipe_kernel(GemmParams<T> p) {
   run_jobs();
 }
 
-template <typename T, int BM, int BN, int WGM, int WGN, int L, int EPI, int MODE, bool SPLIT = false>
+template <typename T, int CFG, int WGM, int WGN, int EPI, int MODE, bool SPLIT = false>
 hipError_t run_pipe(const GemmParams<T>& p, hipStream_t s) {
+  constexpr int BM = kPipeTiles[CFG].bm, BN = kPipeTiles[CFG].bn, L = kPipeTiles[CFG].depth;
   if (EPI != EPI_KEYAD && (p.loss.losses || p.disp.nblk > 0)) return hipErrorInvalidValue;
   if (p.k1 % 64 || p.k2 % 64 || p.n % BN || (EPI == EPI_KEYAD && p.n_key % BN)) return hipErrorInvalidValue;
   if (MODE == PIPE_GRP && (!p.grp_off || p.grp_n < 1 || p.grp_n > 64)) return hipErrorInvalidValue;
@@ -490,7 +491,7 @@ hipError_t run_pipe(const GemmParams<T>& p, hipStream_t s) {
   const int tiles = (MODE == PIPE_GK ? p.gk_n : 1) * ((p.m + BM - 1) / BM + (MODE == PIPE_GRP ? p.grp_n : 0)) *
                     (p.n / BN) * ks;
   if (tiles == 0) return hipSuccess;
-  constexpr int per_cu = 163840 / ((L + 1) * BM * 128 + L * BN * 128);
+  constexpr int per_cu = kPipeTiles[CFG].per_cu;
   GemmParams<T> q = p;
   q.group_m = walk_group_m((p.m + BM - 1) / BM, p.n / BN, BM, BN);
   launch_kernel((pipe_kernel<T, BM, BN, WGM, WGN, L, EPI, MODE, SPLIT>), dim3(std::min(tiles, num_cus() * per_cu)),
@@ -504,22 +505,22 @@ hipError_t run_pipe_cfg(const GemmParams<T>& p, int cfg, hipStream_t s) {
   if constexpr (MODE == PIPE_DENSE) {
     if (p.ksplit > 1) {
       switch (cfg) {
-        case 4: return run_pipe<T, 128, 128, 2, 4, 4, EPI, MODE, true>(p, s);
-        case 6: return run_pipe<T, 128, 64, 4, 2, 3, EPI, MODE, true>(p, s);
-        case 7: return run_pipe<T, 64, 64, 4, 2, 4, EPI, MODE, true>(p, s);
+        case 4: return run_pipe<T, 4, 2, 4, EPI, MODE, true>(p, s);
+        case 6: return run_pipe<T, 6, 4, 2, EPI, MODE, true>(p, s);
+        case 7: return run_pipe<T, 7, 4, 2, EPI, MODE, true>(p, s);
       }
       return hipErrorInvalidValue;
     }
   }
   switch (cfg) {
-    case 0: return run_pipe<T, 256, 256, 2, 4, 2, EPI, MODE>(p, s);
-    case 1: return run_pipe<T, 256, 192, 2, 4, 2, EPI, MODE>(p, s);
-    case 2: return run_pipe<T, 256, 128, 4, 2, 2, EPI, MODE>(p, s);
-    case 3: return run_pipe<T, 128, 192, 2, 4, 3, EPI, MODE>(p, s);
-    case 4: return run_pipe<T, 128, 128, 2, 4, 4, EPI, MODE>(p, s);
-    case 5: return run_pipe<T, 128, 128, 2, 4, 2, EPI, MODE>(p, s);
-    case 6: return run_pipe<T, 128, 64, 4, 2, 3, EPI, MODE>(p, s);
-    case 7: return run_pipe<T, 64, 64, 4, 2, 4, EPI, MODE>(p, s);
+    case 0: return run_pipe<T, 0, 2, 4, EPI, MODE>(p, s);
+    case 1: return run_pipe<T, 1, 2, 4, EPI, MODE>(p, s);
+    case 2: return run_pipe<T, 2, 4, 2, EPI, MODE>(p, s);
+    case 3: return run_pipe<T, 3, 2, 4, EPI, MODE>(p, s);
+    case 4: return run_pipe<T, 4, 2, 4, EPI, MODE>(p, s);
+    case 5: return run_pipe<T, 5, 2, 4, EPI, MODE>(p, s);
+    case 6: return run_pipe<T, 6, 4, 2, EPI, MODE>(p, s);
+    case 7: return run_pipe<T, 7, 4, 2, EPI, MODE>(p, s);
   }
   return hipErrorInvalidValue;
 }

@@ -275,10 +275,39 @@ constexpr bool out_in_ring() {
 template <typename T>
 hipError_t gemm_vs_run(const GemmParams<T>& p, int tile, int epi, bool ext, bool mx, hipStream_t s);
 
-// The pipelined 16-bit tiles (gemm_pipe.h): tile `cfg` of kPipeTiles with the
-// epilogue EPI_STORE (+ the residual where p.resid is set) or EPI_KEYAD (relu²
-// on columns below n_key, the gate mask on the rest); p.k2 > 0: a second K
-// segment; p.ksplit > 1: fp32 partials into p.part.
+// The pipelined 16-bit tiles (gemm_pipe.h) and their times in microseconds, for
+// plan_pipe (gemm.hip): a 64-wide K slice of a tile with nearly every CU busy
+// (`slice`; of two tiles that share a CU: the pair's time over two) and with
+// some idle (`alone`; where two could share a CU, one tile on it), and a tile's
+// start and end (`round`).  Fitted to launches of every tile and K split over
+// 1054 dense products (fp16 and bf16, 66 to 8192 rows, 128 to 8192 columns, K =
+// 512 to 8704), 140 row-group and 70 K-group products: the choice takes 0.25%
+// more than the fastest on average (a fit to bf16 at K = 8192 alone: 2.1%, and
+// up to 44% on a few hundred rows).
+struct PipeTile {
+  int bm, bn, depth;  // depth: slices of B in LDS (one more of A)
+  int per_cu;         // tiles that a CU holds at once
+  double slice, alone, round;
+};
+constexpr PipeTile kPipeTiles[] = {
+    {256, 256, 2, 1, 1.57, 1.27, 3.8}, {256, 192, 2, 1, 1.12, 0.86, 5.2}, {256, 128, 2, 1, 0.85, 0.65, 3.3},
+    {128, 192, 3, 1, 0.62, 0.53, 3.7}, {128, 128, 4, 1, 0.47, 0.42, 2.6}, {128, 128, 2, 2, 0.49, 0.55, 1.2},
+    {128, 64, 3, 1, 0.33, 0.33, 0.8},  {64, 64, 4, 2, 0.21, 0.24, 1.0},
+};
+constexpr int kPipeN = sizeof(kPipeTiles) / sizeof(kPipeTiles[0]);
+// 64 16-bit elements of K are 128 bytes a row, of 160 KB.
+constexpr int pipe_lds_bytes(const PipeTile& t) { return ((t.depth + 1) * t.bm + t.depth * t.bn) * 128; }
+constexpr bool pipe_tiles_fit() {
+  for (const PipeTile& t : kPipeTiles)
+    if (t.per_cu != 163840 / pipe_lds_bytes(t)) return false;
+  return true;
+}
+static_assert(pipe_tiles_fit(), "tiles a CU holds");
+
+// Tile `cfg` of kPipeTiles with the epilogue EPI_STORE (+ the residual where
+// p.resid is set) or EPI_KEYAD (relu² on columns below n_key, the gate mask on
+// the rest); p.k2 > 0: a second K segment; p.ksplit > 1: fp32 partials into
+// p.part.
 enum { PIPE_DENSE = 0, PIPE_GRP = 1, PIPE_GK = 2 };
 template <typename T>
 hipError_t pipe_run(const GemmParams<T>& p, int cfg, int epi, int mode, hipStream_t s);

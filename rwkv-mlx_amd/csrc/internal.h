@@ -36,6 +36,11 @@ struct Probe {
 Probe*& probe_slot();
 // Compute units of the current device (read once per process).
 int num_cus();
+// For the tests: the tile (of kPipeTiles, gemm_tile.h) and K split that a 16-bit
+// product of more than 64 rows runs on; returns the work items that the card
+// holds at once, -1 for arguments that no product has.  mode: PIPE_DENSE (0),
+// PIPE_GRP (1, row groups), PIPE_GK (2, K groups).  Not part of the C ABI.
+int gemm_plan(int mode, int m, int n, int n_key, int k, int groups, int* cfg, int* ks);
 hipError_t mark(hipError_t launched, const char* name, hipStream_t s);
 
 // Every kernel of the library is launched through here (the arguments are

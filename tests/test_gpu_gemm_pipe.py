@@ -1,8 +1,10 @@
 """The pipelined 16-bit products (key with relu², value) at the sizes where
 their tiles, rings and tile choice can go wrong: one K slice per tile (fewer
 than the ring holds) with many tiles per workgroup, ragged last rows, the
-smallest widths, K splits, every tile shape, the K-extension with the residual,
-and row groups that are empty, ragged or hold almost every token."""
+smallest widths, the K-extension with the residual, and row groups that are
+empty, ragged or hold almost every token.  INSTANCES, ROW_GROUPS and K_GROUPS
+reach every tile that the planner can choose, split and unsplit, in every form
+(test_gemm_plan.py holds them to it)."""
 import numpy as np
 import pytest
 
@@ -15,9 +17,25 @@ UNIT = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}
 SHAPES = [(65, 64, 64), (66, 128, 64), (129, 64, 192), (200, 2048, 1024), (200, 512, 8192), (257, 192, 384),
           (300, 320, 576), (1000, 64, 960), (2031, 1024, 3584), (4096, 768, 3072), (4100, 768, 256),
           (8192, 1024, 4096), (9001, 256, 512), (33000, 64, 128), (70000, 64, 64)]
+# (N, C, F): the value product is N x C over K = F, the key product N x F over K = C
+INSTANCES = [(4100, 2048, 64), (4100, 64, 2048), (3000, 3072, 256), (3000, 256, 3072), (513, 8192, 192),
+             (513, 192, 8192), (1474, 3072, 256), (1474, 256, 3072), (700, 3072, 768), (700, 768, 3072),
+             (513, 4096, 64), (513, 64, 4096), (9340, 896, 64), (65, 64, 2048), (65, 2048, 64), (131, 3072, 4096),
+             (131, 4096, 3072), (65, 2048, 4096), (65, 4096, 2048), (200, 2048, 8192)]
+# (N, C, F, E, k, one popular expert)
+ROW_GROUPS = [(3, 64, 64, 2, 1, False), (130, 128, 192, 64, 1, False), (600, 64, 320, 8, 2, True),
+              (3000, 256, 512, 16, 2, True), (20000, 64, 64, 4, 1, True), (2500, 768, 768, 5, 3, False),
+              (3, 320, 64, 1, 1, False), (17, 64, 512, 64, 2, False), (17, 1024, 64, 32, 1, False),
+              (4000, 64, 512, 8, 4, False), (1000, 2048, 128, 4, 4, False), (10000, 128, 192, 64, 4, False),
+              (10000, 192, 128, 64, 4, False), (300, 192, 3072, 4, 4, False), (300, 3072, 192, 4, 4, False),
+              (1000, 192, 576, 64, 4, False), (1000, 576, 192, 64, 4, False), (130, 768, 3072, 8, 4, False),
+              (130, 3072, 768, 8, 4, False)]
+# (N, C, F, E, k): the weight gradients, F x C and C x F for each expert
+K_GROUPS = [(3, 64, 64, 1, 1), (3, 64, 64, 4, 1), (3, 64, 512, 64, 1), (3, 384, 768, 32, 1), (3, 576, 192, 64, 1),
+            (3, 768, 3072, 2, 1), (600, 192, 576, 32, 4), (1500, 768, 384, 8, 4), (2048, 1024, 4096, 8, 2)]
 
 
-@pytest.mark.parametrize("N,C,F", SHAPES)
+@pytest.mark.parametrize("N,C,F", SHAPES + INSTANCES)
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 def test_key_and_value_products(device, dtype, N, C, F):
     import torch
@@ -77,9 +95,7 @@ def test_layer_with_adapter_columns_and_residual(device, dtype, N, C, F, E, k, r
     assert err <= 5 * UNIT[dtype], err
 
 
-@pytest.mark.parametrize("N,C,F,E,k,hot", [(3, 64, 64, 2, 1, False), (130, 128, 192, 64, 1, False),
-                                           (600, 64, 320, 8, 2, True), (3000, 256, 512, 16, 2, True),
-                                           (20000, 64, 64, 4, 1, True), (2500, 768, 768, 5, 3, False)])
+@pytest.mark.parametrize("N,C,F,E,k,hot", ROW_GROUPS)
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 def test_row_groups(device, dtype, N, C, F, E, k, hot):
     """MoE_CMix's grouped products: groups that are empty, ragged, or hold
@@ -137,3 +153,39 @@ def test_row_groups_reduce_the_losses(device, N, C, F, E, k):
     ref_z = torch.logsumexp(lg, -1).square().mean()
     assert abs(aux.item() - ref_aux.item()) <= 1e-6 * ref_aux.item()
     assert abs(z.item() - ref_z.item()) <= 1e-6 * ref_z.item()
+
+
+@pytest.mark.parametrize("N,C,F,E,k", K_GROUPS)
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_k_groups(device, dtype, N, C, F, E, k):
+    """The weight gradients of the full-expert layer, each expert's over its own
+    routed rows, against float64; an expert without rows gets zeros."""
+    import torch
+    from rwkv_mlx_amd import _lib
+    dt = {"f16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    g = torch.Generator(device=device).manual_seed(N + C + F + E)
+    rand = lambda *s, sc=1.0: (torch.randn(*s, generator=g, device=device) * sc).to(dt)
+    x, dO, xk = rand(1, N, C), rand(1, N, C), torch.rand(E, C, generator=g, device=device).to(dt)
+    wk, wv, wg = rand(E, F, C, sc=C ** -0.5), rand(E, C, F, sc=F ** -0.5), rand(E, C)
+    logits = torch.randn(N, E, generator=g, device=device)
+    sel, inds = logits.topk(k, -1)
+    inds = inds.int()
+    desc = _lib.make_desc(1, N, C, F, E, k, 1, dtype)
+    nb = _lib.experts_backward_workspace_bytes(desc)
+    ws = torch.full((nb,), 0xFF, dtype=torch.uint8, device=device)
+    dwk, dwv = torch.full_like(wk, float("nan")), torch.full_like(wv, float("nan"))
+    _lib.experts_backward(desc, ws, nb, _lib.current_stream(device), x=x, x_k=xk, w_key=wk, w_value=wv, w_gate=wg,
+                          logits=logits, inds=inds, d_out=dO, d_w_key=dwk, d_w_value=dwv)
+    torch.cuda.synchronize()
+    gates = sel.double().softmax(-1)
+    xd, dOd = x[0].double(), dO[0].double()
+    mix = torch.cat([torch.zeros_like(xd[:1]), xd[:-1]]) - xd
+    for e in range(E):
+        at, slot = (inds == e).nonzero(as_tuple=True)
+        rows = xd[at] + mix[at] * xk[e].double()
+        p = torch.relu(rows @ wk[e].double().T)
+        gdo = gates[at, slot][:, None] * dOd[at]
+        for got, ref in ((dwk[e], (2 * p * (gdo @ wv[e].double())).T @ rows), (dwv[e], gdo.T @ (p * p))):
+            # the mixed rows, p, h, u, dp, g dO and the gradient each round to dtype
+            err = (got.double() - ref).norm().item()
+            assert err <= 7 * UNIT[dtype] * ref.norm().item(), (e, err)
