@@ -418,11 +418,17 @@ class KernelTimer:
         return [(nm, tot[nm] / len(self.used)) for nm in order]
 
 
+_CUDA_INDEX: dict = {}  # torch.device -> its index, of the CUDA devices asked for so far
+
+
 def current_stream(device) -> int:
     """The hipStream_t of torch's current stream on `device` (anything that
-    torch.cuda.current_stream takes; for a CUDA torch.device without the Stream
-    object that it makes, 2.5 us a call)."""
-    if not isinstance(device, torch.device) or device.type != "cuda":
-        return torch.cuda.current_stream(device).cuda_stream  # (raises for what is no CUDA device)
-    index = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    torch.cuda.current_stream takes; for a CUDA torch.device with an index
+    without the Stream object that it makes, 2.5 us a call)."""
+    index = _CUDA_INDEX.get(device)
+    if index is None:
+        stream = torch.cuda.current_stream(device).cuda_stream  # (raises for what is no CUDA device)
+        if isinstance(device, torch.device) and device.index is not None:
+            _CUDA_INDEX[device] = device.index
+        return stream
+    return torch._C._cuda_getCurrentRawStream(index)
