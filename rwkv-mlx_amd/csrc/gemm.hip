@@ -858,6 +858,18 @@ PipePlan plan_pipe(int mode, int m, int n, int n_key, int nkt, int groups = 1, l
   return best;
 }
 
+// Whether a row-group key product runs this file's 64x64 ring tile instead: four
+// waves with a shorter way in and out, for a few rows whose tiles fit the card at
+// once (64 tokens, 4 experts of 512 x 2048 fp16: 5.6 against 7.1 us; 8 experts of
+// 768 x 3072, top-2: 10.0 / 11.6).  Each of its slices takes longer, and from K =
+// 1024 on it wins or loses with the experts that the rows reach (one token, 16
+// experts of 1024 x 3584, top-4: 47.4 / 45.8 us a forward).
+bool ring_rows(int m, int n, int nkt, int groups, const PipePlan& pp) {
+  const int cus = num_cus();
+  const unsigned tiles = group_tile_rows(m, groups, 64) * (n / 64);
+  return tiles <= 2u * cus && pipe_us(kPipeTiles[7], tiles, nkt, cus) - 2.6 + 0.17 * nkt < pp.us;
+}
+
 // Whether a 16-bit product runs this file's 64-row tiles (codes 8 and 9).
 bool small_rows_plan(const TilePlan& pl) { return pl.t == 8 || pl.t == 9; }
 
@@ -960,10 +972,12 @@ int num_cus() {
 }
 
 int gemm_plan(int mode, int m, int n, int n_key, int k, int groups, int* cfg, int* ks) {
+  const bool rows_key = mode == 3;
+  if (rows_key) mode = PIPE_GRP;
   if (mode < PIPE_DENSE || mode > PIPE_GK || m < 1 || n < 64 || n % 64 || n_key % 64 || k < 64 || groups < 1 || !cfg || !ks)
     return -1;
   const PipePlan p = plan_pipe(mode, m, n, n_key, k / 64, groups);
-  *cfg = p.cfg;
+  *cfg = rows_key && p.cfg >= 0 && ring_rows(m, n, k / 64, groups, p) ? kPipeN : p.cfg;
   *ks = p.ks;
   return p.cfg < 0 ? -1 : kPipeTiles[p.cfg].per_cu * num_cus();
 }
@@ -1117,7 +1131,7 @@ hipError_t launch_cmix_value_sparse(int dtype, const void* h, const void* wv, in
   return mark(e, "cmix_value_sparse", s);
 }
 
-// Grouped product.  16-bit: the pipelined tiles; fp32: one tile per workgroup,
+// Grouped product.  16-bit: the pipelined tiles (a few rows' key product: a ring tile); fp32: one tile per workgroup,
 // 128x128 or 64x64 by waves x operand rows per tile (ceil(tiles / CUs) x (BM +
 // BN): these products are bound by each CU's operand loads, and a partial
 // last wave costs as much as a full one), ties to the larger.
@@ -1126,6 +1140,9 @@ hipError_t dispatch_grouped(const GemmParams<T>& p, hipStream_t s) {
   if constexpr (sizeof(T) == 2) {
     const PipePlan pp = plan_pipe(PIPE_GRP, p.m, p.n, p.n, p.k1 / 64, p.grp_n);
     if (pp.cfg < 0) return hipErrorInvalidValue;
+    if constexpr (EPI == EPI_KEY)
+      if (ring_rows(p.m, p.n, p.k1 / 64, p.grp_n, pp))
+        return run<T, 64, 64, 2, 2, 3, EPI, false, 32, 0, 128, false, false, true>(p, s, false);
     return pipe_run<T>(p, pp.cfg, EPI == EPI_KEY ? EPI_KEYAD : EPI_STORE, PIPE_GRP, s);
   } else {
     const int cus = num_cus();

@@ -39,7 +39,8 @@ int num_cus();
 // For the tests: the tile (of kPipeTiles, gemm_tile.h) and K split that a 16-bit
 // product of more than 64 rows runs on; returns the work items that the card
 // holds at once, -1 for arguments that no product has.  mode: PIPE_DENSE (0),
-// PIPE_GRP (1, row groups), PIPE_GK (2, K groups).  Not part of the C ABI.
+// PIPE_GRP (1, row groups; 3, their key product, whose cfg kPipeN is the ring
+// tile), PIPE_GK (2, K groups).  Not part of the C ABI.
 int gemm_plan(int mode, int m, int n, int n_key, int k, int groups, int* cfg, int* ks);
 hipError_t mark(hipError_t launched, const char* name, hipStream_t s);
 

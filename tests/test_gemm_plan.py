@@ -7,10 +7,12 @@ import pytest
 
 import test_gpu_gemm_pipe as P
 
-DENSE, ROWS, KS = 0, 1, 2
-# tiles of gemm_tile.h's kPipeTiles; three of them also split K
+DENSE, ROWS, KS, ROWS_KEY = 0, 1, 2, 3
+# tiles of gemm_tile.h's kPipeTiles; three of them also split K.  A row-group key
+# product can also run the 64x64 ring tile.
 TILES = ((256, 256), (256, 192), (256, 128), (128, 192), (128, 128), (128, 128), (128, 64), (64, 64))
 SPLIT = (4, 6, 7)
+RING = len(TILES)
 
 
 @pytest.fixture(scope="module")
@@ -61,11 +63,11 @@ def test_gpu_shapes_reach_every_kernel(plan):
         value.add(form(plan(DENSE, N, C, F)))
         key.add(form(plan(DENSE, N, F, C)))
     for N, C, F, E, k, _ in P.ROW_GROUPS:
-        rows_key.add(plan(ROWS, N * k, F, C, E)[0])
+        rows_key.add(plan(ROWS_KEY, N * k, F, C, E)[0])
         rows_value.add(plan(ROWS, N * k, C, F, E)[0])
     for N, C, F, E, k in P.K_GROUPS:
         avg = max(1, (N * k + 128 * E + 127) // 128 * 128 // E // 64) * 64
         kgroups |= {plan(KS, F, C, avg, E)[0], plan(KS, C, F, avg, E)[0]}
     every = set(range(len(TILES)))
     assert value == key == {(c, False) for c in every} | {(c, True) for c in SPLIT}
-    assert rows_key == rows_value == kgroups == every
+    assert rows_key == every | {RING} and rows_value == kgroups == every
