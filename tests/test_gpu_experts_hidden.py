@@ -42,3 +42,31 @@ def test_gradients_and_each_weight_alone(layer):
     for name in ("d_w_key", "d_w_value", "d_w_gate"):
         alone = layer.backward((name,))[name]
         assert np.array_equal(B._bits(alone), B._bits(got[name])), name
+
+
+def test_more_token_tiles_than_a_second_grid_dimension(device):
+    """Frozen expert weights and more than 65535 tiles of 64 routed rows: dx of
+    the last sequences is that of these sequences alone."""
+    import torch
+    from rwkv_mlx_amd import _lib
+    Bn, T, C, F, E, k = 65600, 32, 64, 64, 2, 2
+    g = torch.Generator(device=device).manual_seed(7)
+    rand = lambda *s, sc=1.0: (torch.randn(*s, generator=g, device=device) * sc).half()
+    x, dO, xk = rand(Bn, T, C), rand(Bn, T, C), torch.rand(E, C, generator=g, device=device).half()
+    wk, wv, wg = rand(E, F, C, sc=C ** -0.5), rand(E, C, F, sc=F ** -0.5), rand(E, C)
+    logits = torch.randn(Bn * T, E, generator=g, device=device)
+    inds = logits.topk(k, -1)[1].int()
+
+    def dx(at):
+        n = Bn - at
+        desc = _lib.make_desc(n, T, C, F, E, k, 1, "f16")
+        nb = _lib.experts_backward_workspace_bytes(desc)
+        ws = torch.full((nb,), 0xFF, dtype=torch.uint8, device=device)
+        out = torch.full((n, T, C), float("nan"), dtype=torch.float16, device=device)
+        _lib.experts_backward(desc, ws, nb, _lib.current_stream(device), x=x[at:], x_k=xk, w_key=wk, w_value=wv,
+                              w_gate=wg, logits=logits[at * T:], inds=inds[at * T:], d_out=dO[at:], d_x=out)
+        torch.cuda.synchronize()
+        return out
+    whole, last = dx(0), dx(Bn - 40)
+    assert torch.isfinite(whole).all()
+    assert (whole[-40:].double() - last.double()).norm() <= 4 * 2.0 ** -11 * last.double().norm()

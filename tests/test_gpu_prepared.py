@@ -114,3 +114,21 @@ def test_module_cache_follows_updates(device):
         m.invalidate_prepared()
         f, _, _ = m(x)
         assert torch.equal(f, fresh_out()) and not torch.equal(e, f)
+
+
+def test_module_cache_follows_the_parameters_device():
+    """A layer whose parameters move to the host between two calls on the same
+    input (no version counter moves) gives the same bits."""
+    import torch
+    from rwkv_mlx_amd.moe import build_layer
+    torch.manual_seed(2)
+    m = build_layer(768, 3072, 8, 2, 16).cuda().half()
+    with torch.no_grad():
+        m.base.x_k.uniform_(0, 1)
+        m.lora_B.normal_(0, 0.02)
+        for shape in ((2, 300, 768), (8, 1, 768)):  # (the second reads the base weights' decode layout)
+            x = torch.randn(*shape, device="cuda").half()
+            a, _, _ = m.cuda()(x)
+            b, _, _ = m.cpu()(x)
+            c, _, _ = m.cuda()(x)
+            assert torch.equal(a, b) and torch.equal(a, c)
