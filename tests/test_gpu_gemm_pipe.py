@@ -29,7 +29,8 @@ ROW_GROUPS = [(3, 64, 64, 2, 1, False), (130, 128, 192, 64, 1, False), (600, 64,
               (4000, 64, 512, 8, 4, False), (1000, 2048, 128, 4, 4, False), (10000, 128, 192, 64, 4, False),
               (10000, 192, 128, 64, 4, False), (300, 192, 3072, 4, 4, False), (300, 3072, 192, 4, 4, False),
               (1000, 192, 576, 64, 4, False), (1000, 576, 192, 64, 4, False), (130, 768, 3072, 8, 4, False),
-              (130, 3072, 768, 8, 4, False)]
+              (130, 3072, 768, 8, 4, False), (4000, 64, 768, 8, 4, False), (10000, 64, 576, 8, 2, False),
+              (4000, 768, 64, 8, 4, False), (10000, 576, 64, 8, 2, False)]
 # (N, C, F, E, k): the weight gradients, F x C and C x F for each expert
 K_GROUPS = [(3, 64, 64, 1, 1), (3, 64, 64, 4, 1), (3, 64, 512, 64, 1), (3, 384, 768, 32, 1), (3, 576, 192, 64, 1),
             (3, 768, 3072, 2, 1), (600, 192, 576, 32, 4), (1500, 768, 384, 8, 4), (2048, 1024, 4096, 8, 2)]
