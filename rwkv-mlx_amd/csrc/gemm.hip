@@ -909,7 +909,7 @@ hipError_t dispatch_tile(const GemmParams<T>& p, hipStream_t s, const TilePlan* 
   if (deferred) *deferred = 1;
   if constexpr (MX) {
     if (vs_enabled() && t == 6) {
-      const hipError_t e = gemm_vs_run<T>(p, t, EPI, EXT, MX, s);
+      const hipError_t e = gemm_vs_run<T>(p, EPI, EXT, MX, s);
       if (e != hipErrorNotSupported) return e;
     }
   } else if constexpr (sizeof(T) == 2) {
@@ -1089,24 +1089,30 @@ hipError_t launch_cmix_value(int dtype, const void* h, const void* wv, int F, co
   return hipSuccess;
 }
 
+// The fused combine runs one 128x96 tile a workgroup, ahead of the pipelined
+// product and the combine launch where those tiles give nearly every CU one and
+// none two: 4096 tokens of 768 x 3072 fp16 25.8 us against 23.4 + 5.2 (the layer
+// 76.6 / 80.2), 2048 of 1536 x 6144 44.3 against 42.3 + 5.1.  A second round, and
+// the 256x128 tile that wider layers took, lose: 6000 x 768 47.2 / 28.6 + 6.6 (the
+// layer 110.3 / 99.8), 8192 x 1024 x 4096 76.9 / 54.1 + 16.0 (230.6 / 223.9), 6000 x
+// 2048 x 8192 bf16 242 / 175 + 17 (458 / 414).
 bool value_combine_fusable(int dtype, int N, int C, int F, int k) {
-  if (dtype == 0 || k < 1 || k > kCombineMaxK || !vs_enabled()) return false;
-  const TilePlan pl = plan_tiles(2, EPI_STORE, N, C, C, F);
-  return (pl.t == 6 && F % 128 == 0 && C % 96 == 0) || (pl.t == 5 && F % 64 == 0 && C % 128 == 0);
+  if (dtype == 0 || k < 1 || k > kCombineMaxK || !vs_enabled() || F % 128 || C % 96) return false;
+  const int cus = num_cus(), tiles = (N + 127) / 128 * (C / 96);
+  return tiles <= cus && tiles * 10 >= cus * 9;
 }
 
 hipError_t launch_cmix_value_combine(int dtype, const void* h, const void* wv, int F, const void* rows,
                                      const int* inds, const void* gates, const void* resid, void* out, int N, int C,
                                      int k, hipStream_t s) {
   if (!value_combine_fusable(dtype, N, C, F, k)) return hipErrorInvalidValue;
-  const TilePlan pl = plan_tiles(2, EPI_STORE, N, C, C, F);
   auto go = [&](auto tag) {
     typedef decltype(tag) T;
     GemmParams<T> p = blank<T>();
     p.a1 = (const T*)h; p.lda1 = F; p.b1 = (const T*)wv; p.ldb1 = F; p.k1 = F;
     p.m = N; p.n = C; p.out = (T*)out; p.ldo = C; p.resid = (const T*)resid;
     p.cmb_rows = (const T*)rows; p.cmb_inds = inds; p.cmb_gates = (const T*)gates; p.cmb_k = k;
-    return gemm_vs_run<T>(p, pl.t, EPI_COMBINE, false, false, s);
+    return gemm_vs_run<T>(p, EPI_COMBINE, false, false, s);
   };
   const hipError_t e = dtype == 1 ? go(f16{}) : go(bf16{});
   return mark(e, "cmix_value_combine", s);
@@ -1135,7 +1141,7 @@ hipError_t launch_cmix_value_sparse(int dtype, const void* h, const void* wv, in
     p.m = N; p.n = C; p.out = (T*)out; p.ldo = C; p.resid = (const T*)resid;
     p.cmb_inds = inds; p.cmb_gates = (const T*)gates; p.cmb_k = k;
     p.n_experts = E; p.rank = r;
-    return gemm_vs_run<T>(p, 6, EPI_SPARSE, true, false, s);
+    return gemm_vs_run<T>(p, EPI_SPARSE, true, false, s);
   };
   const hipError_t e = dtype == 1 ? go(f16{}) : go(bf16{});
   return mark(e, "cmix_value_sparse", s);

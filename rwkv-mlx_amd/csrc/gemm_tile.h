@@ -273,7 +273,7 @@ constexpr bool out_in_ring() {
 // The VGPR-staged form of tile code `tile` (gemm_vs.hip), or
 // hipErrorNotSupported when that tile has none.
 template <typename T>
-hipError_t gemm_vs_run(const GemmParams<T>& p, int tile, int epi, bool ext, bool mx, hipStream_t s);
+hipError_t gemm_vs_run(const GemmParams<T>& p, int epi, bool ext, bool mx, hipStream_t s);
 
 // The pipelined 16-bit tiles (gemm_pipe.h) and their times in microseconds, for
 // plan_pipe (gemm.hip): a 64-wide K slice of a tile with nearly every CU busy

@@ -507,36 +507,30 @@ hipError_t run_vs(const GemmParams<T>& p, hipStream_t s) {
 
 }  // namespace
 
-// Variant of a tile code (gemm.hip's numbering) in the VGPR-staged form;
-// hipErrorNotSupported when there is none (the caller keeps the ring form).
-//   6: 128x96, 4 MFMA waves (2x2, 16x16 blocks), 12 load waves, 256-byte
-//      slices, two in flight per load lane (three and more measured slower):
-//      the SPARSE layer's value products (rank slices, fused combine) and the
-//      fp32-adapter product
-//   5: 256x128, 8 MFMA waves (4x2, 32x32 blocks), 8 load waves, 128-byte
-//      slices: the fused combine of wider layers
+// The VGPR-staged products: the SPARSE layer's value products (rank slices,
+// fused combine) and the fp32-adapter product.  128x96 tiles, 4 MFMA waves (2x2,
+// 16x16 blocks), 12 load waves, 256-byte slices, two in flight per load lane
+// (three and more measured slower).  hipErrorNotSupported for what it does not
+// take (the caller keeps the ring form).
 template <typename T>
-hipError_t gemm_vs_run(const GemmParams<T>& p, int tile, int epi, bool ext, bool mx, hipStream_t s) {
+hipError_t gemm_vs_run(const GemmParams<T>& p, int epi, bool ext, bool mx, hipStream_t s) {
   if constexpr (sizeof(T) != 2) {
     return hipErrorNotSupported;
   } else {
-    if (tile == 5 && !mx && !ext && epi == EPI_COMBINE && p.k1 % 64 == 0)
-      return run_vs<T, 256, 128, 4, 2, 32, 8, 128, 2, EPI_COMBINE, false, false>(p, s);
-    if (tile == 6 && (p.k1 % 128 == 0) && (!ext || p.k2 % 128 == 0)) {
-      if (mx) {
-        if (epi == EPI_RESID) return run_vs<T, 128, 96, 2, 2, 16, 12, 256, 2, EPI_RESID, true, true>(p, s);
-        if (epi == EPI_STORE) return run_vs<T, 128, 96, 2, 2, 16, 12, 256, 2, EPI_STORE, true, true>(p, s);
-        return hipErrorNotSupported;
-      }
-      if (ext && epi == EPI_SPARSE) return run_vs<T, 128, 96, 2, 2, 16, 12, 256, 2, EPI_SPARSE, true, false>(p, s);
-      if (!ext && epi == EPI_COMBINE) return run_vs<T, 128, 96, 2, 2, 16, 12, 256, 2, EPI_COMBINE, false, false>(p, s);
+    if (p.k1 % 128 || (ext && p.k2 % 128)) return hipErrorNotSupported;
+    if (mx) {
+      if (epi == EPI_RESID) return run_vs<T, 128, 96, 2, 2, 16, 12, 256, 2, EPI_RESID, true, true>(p, s);
+      if (epi == EPI_STORE) return run_vs<T, 128, 96, 2, 2, 16, 12, 256, 2, EPI_STORE, true, true>(p, s);
+      return hipErrorNotSupported;
     }
+    if (ext && epi == EPI_SPARSE) return run_vs<T, 128, 96, 2, 2, 16, 12, 256, 2, EPI_SPARSE, true, false>(p, s);
+    if (!ext && epi == EPI_COMBINE) return run_vs<T, 128, 96, 2, 2, 16, 12, 256, 2, EPI_COMBINE, false, false>(p, s);
     return hipErrorNotSupported;
   }
 }
 
-template hipError_t gemm_vs_run<f16>(const GemmParams<f16>&, int, int, bool, bool, hipStream_t);
-template hipError_t gemm_vs_run<bf16>(const GemmParams<bf16>&, int, int, bool, bool, hipStream_t);
-template hipError_t gemm_vs_run<float>(const GemmParams<float>&, int, int, bool, bool, hipStream_t);
+template hipError_t gemm_vs_run<f16>(const GemmParams<f16>&, int, bool, bool, hipStream_t);
+template hipError_t gemm_vs_run<bf16>(const GemmParams<bf16>&, int, bool, bool, hipStream_t);
+template hipError_t gemm_vs_run<float>(const GemmParams<float>&, int, bool, bool, hipStream_t);
 
 }  // namespace rwkvmoe

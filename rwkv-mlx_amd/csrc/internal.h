@@ -158,8 +158,8 @@ hipError_t launch_cmix_value(int dtype, const void* h, const void* wv, int F, co
 // out = round(h·W_valueᵀ + δ) (+ residual), δ from the adapter rows in
 // assignment order (launch_combine with inv NULL), so the base never goes
 // to memory and no combine launch follows.  16-bit layers with 16-bit rows,
-// k <= kCombineMaxK, and a value plan with a VGPR-staged tile
-// (value_combine_fusable); else hipErrorInvalidValue.
+// k <= kCombineMaxK, and about one 128x96 tile a CU (value_combine_fusable);
+// else hipErrorInvalidValue.
 bool value_combine_fusable(int dtype, int N, int C, int F, int k);
 hipError_t launch_cmix_value_combine(int dtype, const void* h, const void* wv, int F, const void* rows,
                                      const int* inds, const void* gates, const void* resid, void* out, int N, int C,

@@ -96,6 +96,38 @@ def test_layer_with_adapter_columns_and_residual(device, dtype, N, C, F, E, k, r
     assert err <= 5 * UNIT[dtype], err
 
 
+@pytest.mark.parametrize("N,C,F,E,k", [(3584, 768, 256, 16, 2), (3585, 768, 256, 16, 2), (4096, 768, 384, 16, 1),
+                                       (4097, 768, 256, 16, 2), (2048, 1536, 256, 16, 4), (2049, 1536, 192, 16, 2)])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_sparse_combine_at_one_tile_a_cu(device, dtype, N, C, F, E, k):
+    """The SPARSE layer on both sides of the range in which the combine runs in
+    the value product's epilogue (231 to 256 tiles of 128x96, F % 128 == 0), token
+    by token against float64."""
+    import torch
+    from rwkv_mlx_amd.moe import build_layer
+    dt = {"f16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    torch.manual_seed(N + F)
+    m = build_layer(C, F, E, k, 16).to(device=device, dtype=dt).requires_grad_(False)
+    m.base.x_k.uniform_(0, 1)
+    m.lora_A.normal_(0, C ** -0.5)
+    m.lora_B.normal_(0, 0.3)
+    x = torch.randn(1, N, C, device=device).to(dt)
+    res = torch.randn(1, N, C, device=device).to(dt)
+    ex = {}
+    with torch.no_grad():
+        out = m(x, residual=res, mode="sparse", extras=ex)[0]
+    xd = x[0].double()
+    sh = torch.cat([torch.zeros_like(xd[:1]), xd[:-1]])
+    ref = res[0].double() + torch.relu((xd + (sh - xd) * m.base.x_k.double().reshape(-1)) @ m.base.key.weight.double().T) \
+        ** 2 @ m.base.value.weight.double().T
+    w = torch.zeros(N, E, dtype=torch.float64, device=device).scatter(1, ex["inds"].long(), ex["gates"].double())
+    for e in range(E):
+        ref += w[:, e:e + 1] * (xd @ m.lora_A[e].double() @ m.lora_B[e].double())
+    err = ((out[0].double() - ref).norm(dim=1) / ref.norm(dim=1)).max().item()
+    # the mix, h, the adapter rows, the base, their sum and the residual's each round to dtype
+    assert err <= 6 * UNIT[dtype], err
+
+
 @pytest.mark.parametrize("N,C,F,E,k,hot", ROW_GROUPS)
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 def test_row_groups(device, dtype, N, C, F, E, k, hot):
