@@ -14,7 +14,8 @@
 //
 // 16-bit products run the pipelined tiles of gemm_pipe.h (planned here,
 // plan_pipe); this file's kernel keeps fp32 products, the fp16 layer with fp32
-// adapters (MX) and 16-bit products of at most 64 rows.
+// adapters (MX), 16-bit products of at most 64 rows and the grouped key product of
+// a few rows (ring_rows).
 //
 // Kernel structure (BM x BN tile, WGM x WGN waves and LW load-only waves):
 //   * K is walked in slices of RB bytes per row that buffer_load_dwordx4 ... lds
@@ -29,8 +30,6 @@
 //     of tiles walked in groups of M-tiles (walk_group_m picks the group
 //     size per launch), so its resident tiles share operands in that XCD's
 //     L2.
-#include <stdlib.h>
-
 #include <algorithm>
 #include <type_traits>
 
@@ -70,8 +69,8 @@ namespace {
 // [B_hi | B_lo' | B_hi] then adds the fp32 delta (moe.py:138-147), and the
 // tile leaves in fp32 (out = base + delta in MLX's promoted dtype), with
 // the residual added in fp32.
-template <typename T, int BM, int BN, int WGM, int WGN, int S, int EPI, bool EXT, int MN, int LW, int RB, bool NTS,
-          bool SPLIT, bool GRP, bool MX, bool GK = false>
+template <typename T, int BM, int BN, int WGM, int WGN, int S, int EPI, bool EXT, int MN, int LW, int RB, bool SPLIT,
+          bool GRP, bool MX, bool GK = false>
 __global__ __launch_bounds__(64 * (WGM * WGN + LW)) void gemm_kernel(GemmParams<T> p) {
   static_assert(!MX || (EXT && !SPLIT && !GRP && (EPI == EPI_STORE || EPI == EPI_RESID)), "mixed value product");
   static_assert(!GK || (!EXT && !SPLIT && !GRP && !MX && EPI == EPI_STORE), "grouped-K product");
@@ -454,8 +453,7 @@ __global__ __launch_bounds__(64 * (WGM * WGN + LW)) void gemm_kernel(GemmParams<
       T* dstp = (EPI == EPI_KEYAD && adapter)
                     ? p.out_ad + (size_t)gm * (p.n - p.n_key) + (n0 - p.n_key) + c
                     : p.out + (GK ? (size_t)g_e * p.gk_ostride : 0) + (size_t)gm * p.ldo + n0 + c;
-      if constexpr (NTS) __builtin_nontemporal_store(v, (u32x4*)dstp);
-      else *(u32x4*)dstp = v;
+      *(u32x4*)dstp = v;
     }
   };
   // split-K epilogue (MFMA waves): the raw fp32 accumulators of this work
@@ -659,7 +657,7 @@ __global__ __launch_bounds__(256) void shift_mix_kernel(const T* __restrict__ x,
 
 
 template <typename T, int BM, int BN, int WGM, int WGN, int S, int EPI, bool EXT, int MN = 32, int LW = 0, int RB = 128,
-          bool NTS = false, bool SPLIT = false, bool GRP = false, bool MX = false, bool GK = false>
+          bool SPLIT = false, bool GRP = false, bool MX = false, bool GK = false>
 hipError_t run(const GemmParams<T>& p, hipStream_t s, bool persistent) {
   typedef typename std::conditional<MX, float, T>::type OT;
   constexpr int BK = RB / (int)sizeof(T);
@@ -685,69 +683,29 @@ hipError_t run(const GemmParams<T>& p, hipStream_t s, bool persistent) {
   }
   GemmParams<T> q = p;
   if (!GRP && !GK && ks == 1) q.group_m = walk_group_m((p.m + BM - 1) / BM, p.n / BN, BM, BN);
-  launch_kernel((gemm_kernel<T, BM, BN, WGM, WGN, S, EPI, EXT, MN, LW, RB, NTS, SPLIT, GRP, MX, GK>),
+  launch_kernel((gemm_kernel<T, BM, BN, WGM, WGN, S, EPI, EXT, MN, LW, RB, SPLIT, GRP, MX, GK>),
                      dim3(grid), dim3(64 * (WGM * WGN + LW)), 0, s, q);
   return hipGetLastError();
 }
 
-// Tile codes: 0 = automatic, 1 = 128x128 persistent, 2 = 128x64 persistent,
-// 3 = 256x192 (8 waves), 5 = 256x128 (8 waves), 6 = 128x96 (16x16 MFMA),
-// 7 = 64-row tiles with K split (as for small products), 8 = 64x16 tiles over
-// the whole K (16-bit, at most 64 rows), 9 = 64x16 tiles with K split,
-// 10 = 256x256 (8 waves of 128x64, 64-byte K slices, 5 stages; 16-bit; the
-// relu² key products with 128-byte slices in 2 stages).
-// Only a tuning build (-DRWKVMOE_TUNING) lets RWKVMOE_GEMM_TILE force a code;
-// the library as built reads no environment and always plans automatically.
-int tile_override() {
-#ifdef RWKVMOE_TUNING
-  static int v = [] {
-    const char* s = getenv("RWKVMOE_GEMM_TILE");
-    return s ? atoi(s) : 0;
-  }();
-  return v;
-#else
-  return 0;
-#endif
-}
-
-// Whether the 256x192 and 128x96 tiles run in their VGPR-staged form
-// (gemm_vs.hip).  Only a tuning build (-DRWKVMOE_TUNING) lets RWKVMOE_VS=0
-// select the global_load_lds ring form instead, for A/B timing.
-bool vs_enabled() {
-#ifdef RWKVMOE_TUNING
-  static int v = [] {
-    const char* s = getenv("RWKVMOE_VS");
-    return s ? atoi(s) : 1;
-  }();
-  return v != 0;
-#else
-  return true;
-#endif
-}
-
-// Automatic choice (16-bit): the largest tile that still gives every CU a
-// tile — operand traffic from L2 per FLOP falls as 1/BM + 1/BN, and L2->CU
-// bandwidth, not MFMA issue, bounds these products.
-//   256x256 (8 waves) when N % 256 == 0 and it yields >= 2 tiles per CU with
-//   a last wave at least half full (the wide layers' products: 556 / 518
-//   against 732 / 706 us for the 256x128 ring at 16384 x 8192 x 2048 and
-//   16384 x 2048 x 8192 bf16),
-//   256x192 (8 waves) when N % 192 == 0 and it yields >= 90% of a tile per CU,
-//   256x128 (8 waves) when N % 128 == 0 and it yields >= 1 tile per CU,
-//   128x96 (16x16 MFMA blocks, 256-byte K slices, 4 MFMA waves + 10 waves that
-//   only issue loads: DMA throughput grows with the number of issuing waves)
-//   when N % 96 == 0 and it yields ~1 tile per CU,
-//   else persistent 128x128 (N % 128 == 0) or 128x64.
-// When that leaves more than half of the CUs idle (decode batches, small
-// layers): 64-row tiles (x128 for 16-bit types when N allows, else x64), and
-// K split into the most work items per tile that keeps them within 1.25 per
-// CU and at least 2 K slices each (the partials are reduced by
-// splitk_reduce_kernel in a fixed order) — except 16-bit products of at most
-// 64 rows whose 64x16 tiles give half a wave: those run unsplit.
+// The tiles of this file's kernel.  Codes: 1 = 128x128 and 2 = 128x64 (both
+// persistent), 6 = 128x96 (16x16 MFMA), 7 = 64x64 with K split, 8 = 64x16 over the
+// whole K (16-bit, at most 64 rows), 9 = 64x16 with K split.
+//   fp32: 128x128 where n allows, else 128x64; where that leaves more than half of
+//   the CUs idle, 64x64, and K split into the most work items per tile that keeps
+//   them within 1.25 per CU and at least 2 K slices each (the partials are reduced
+//   by splitk_reduce_kernel in a fixed order).
+//   16-bit: at most 64 rows run 64x16 tiles where the others would leave more than
+//   half of the CUs idle: unsplit where they give half a wave (no partials, no
+//   reduction launch), else with K split, which for the same fill writes 8x fewer
+//   partials than 64x128 tiles.  The mixed product (MX) and the SPARSE value
+//   product with rank slices take 128x96 where 256-row tiles do not fill the chip
+//   and 128x96 tiles do (at least 90%); the mixed product else 128x128 or 128x64,
+//   and neither runs where the plan is one of 64-row tiles.  Other 16-bit products
+//   have the pipelined tiles' plan (plan_pipe), whatever code this gives them.
 struct TilePlan {
-  int t;   // tile code (RWKVMOE_GEMM_TILE numbering)
-  int bn;  // t == 7: tile width
-  int ks;  // t == 7: work items per tile
+  int t;   // tile code
+  int ks;  // t == 7 or 9: work items per tile
 };
 
 TilePlan plan_tiles(int elem, int epi, int m, int n, int n_key, int k_total) {
@@ -755,49 +713,28 @@ TilePlan plan_tiles(int elem, int epi, int m, int n, int n_key, int k_total) {
   // a tile never straddles the key / adapter column boundary
   auto fits = [&](int bn) { return n % bn == 0 && (epi != EPI_KEYAD || n_key % bn == 0); };
   auto tiles = [&](int bm, int bn) { return ((m + bm - 1) / bm) * (n / bn); };
-  TilePlan pl{tile_override(), 0, 1};
-  const bool automatic = pl.t == 0;
-  if (automatic) {
-    // (the adapter epilogue's extra live values do not fit 256x192's register budget)
-    // 256x256 for products of two or more waves of such tiles whose last wave
-    // is at least half full: half the LDS reads per FLOP of the 64x64 wave
-    // tiles (8 waves of 128x64)
-    const int t256 = tiles(256, 256);
-    if (elem == 2 && fits(256) && k_total % 32 == 0 && t256 >= 2 * cus && (t256 % cus == 0 || 2 * (t256 % cus) >= cus))
-      pl.t = 10;
-    else if (elem == 2 && epi != EPI_KEYAD && fits(192) && tiles(256, 192) * 10 >= cus * 9) pl.t = 3;
-    else if (elem == 2 && fits(128) && tiles(256, 128) >= cus) pl.t = 5;
-    else if (elem == 2 && fits(96) && tiles(128, 96) * 10 >= cus * 9) pl.t = 6;
-    else pl.t = fits(128) ? 1 : 2;
-    const int chosen = pl.t == 10 ? t256 : pl.t == 3 ? tiles(256, 192) : pl.t == 5 ? tiles(256, 128)
-                     : pl.t == 6 ? tiles(128, 96) : pl.t == 1 ? tiles(128, 128) : tiles(128, 64);
-    if (chosen * 2 <= cus) pl.t = 7;
-  }
-  if (pl.t == 7) {
-    pl.bn = (elem == 2 && fits(128)) ? 128 : 64;
-    const int nkt = k_total / (128 / elem);  // K slices of 128 bytes
-    const int ts = tiles(64, pl.bn);
-    if (ts * 2 <= cus)
-      for (int c = 2; c <= nkt; ++c)
-        if (nkt % c == 0 && nkt / c >= 2 && ts * c <= cus + cus / 4) pl.ks = c;
-    // a few rows (decode batches): 64x16 tiles over the whole K when they
-    // give at least half a wave, so no split partials and no reduction
-    // launch; else 64x16 tiles with K split, which for the same fill write
-    // 8x fewer partials than 64x128 tiles
-    if (automatic && elem == 2 && m <= 64 && fits(16)) {
-      const int t16 = tiles(64, 16);
-      if (t16 * 2 >= cus) {
-        pl.t = 8;
-        pl.ks = 1;
-      } else {
-        int c16 = 1;
-        for (int c = 2; c <= nkt; ++c)
-          if (nkt % c == 0 && nkt / c >= 2 && t16 * c <= cus + cus / 4) c16 = c;
-        if (c16 > 1) {
-          pl.t = 9;
-          pl.ks = c16;
-        }
-      }
+  const bool wide = elem == 2 && ((epi != EPI_KEYAD && fits(192) && tiles(256, 192) * 10 >= cus * 9) ||
+                                  (fits(128) && tiles(256, 128) >= cus));
+  TilePlan pl{fits(128) ? 1 : 2, 1};
+  if (elem == 2 && !wide && fits(96) && tiles(128, 96) * 10 >= cus * 9) pl.t = 6;
+  const int chosen = pl.t == 6 ? tiles(128, 96) : pl.t == 1 ? tiles(128, 128) : tiles(128, 64);
+  if (chosen * 2 > cus) return pl;
+  const int nkt = k_total / (128 / elem);  // K slices of 128 bytes
+  auto split = [&](int items) {
+    int ks = 1;
+    for (int c = 2; c <= nkt; ++c)
+      if (nkt % c == 0 && nkt / c >= 2 && items * c <= cus + cus / 4) ks = c;
+    return ks;
+  };
+  pl.t = 7;
+  if (elem == 4) {
+    if (tiles(64, 64) * 2 <= cus) pl.ks = split(tiles(64, 64));
+  } else if (m <= 64 && fits(16)) {
+    const int t16 = tiles(64, 16);
+    if (t16 * 2 >= cus) {
+      pl.t = 8;
+    } else if ((pl.ks = split(t16)) > 1) {
+      pl.t = 9;
     }
   }
   return pl;
@@ -889,7 +826,7 @@ bool small_rows_plan(const TilePlan& pl) { return pl.t == 8 || pl.t == 9; }
 template <typename T, int BM, int BN, int EPI, bool EXT, int LW = 0, int WGM = 2, int WGN = 2, int MN = 32>
 hipError_t run_small(GemmParams<T> p, int ks, hipStream_t s, int* deferred) {
   p.ksplit = ks;
-  const hipError_t e = run<T, BM, BN, WGM, WGN, 3, EPI, EXT, MN, LW, 128, false, true>(p, s, false);
+  const hipError_t e = run<T, BM, BN, WGM, WGN, 3, EPI, EXT, MN, LW, 128, true>(p, s, false);
   if (deferred) *deferred = ks > 1 ? ks : 1;
   if (e != hipSuccess || ks <= 1 || deferred) return e;
   const int grid = (p.m * (p.n / 4) + 255) / 256;
@@ -897,8 +834,8 @@ hipError_t run_small(GemmParams<T> p, int ks, hipStream_t s, int* deferred) {
   return hipGetLastError();
 }
 
-// Tile codes a mixed value product (MX) runs: the unsplit 16-bit tiles.
-bool mixed_tile_ok(int t) { return t == 1 || t == 2 || t == 3 || t == 5 || t == 6 || t == 10; }
+// Tile codes a mixed value product (MX) runs.
+bool mixed_tile_ok(int t) { return t == 1 || t == 2 || t == 6; }
 
 template <typename T, int EPI, bool EXT, bool MX = false>
 hipError_t dispatch_tile(const GemmParams<T>& p, hipStream_t s, const TilePlan* given = nullptr,
@@ -908,7 +845,7 @@ hipError_t dispatch_tile(const GemmParams<T>& p, hipStream_t s, const TilePlan* 
   const int t = pl.t;
   if (deferred) *deferred = 1;
   if constexpr (MX) {
-    if (vs_enabled() && t == 6) {
+    if (t == 6) {
       const hipError_t e = gemm_vs_run<T>(p, EPI, EXT, MX, s);
       if (e != hipErrorNotSupported) return e;
     }
@@ -929,24 +866,22 @@ hipError_t dispatch_tile(const GemmParams<T>& p, hipStream_t s, const TilePlan* 
     return hipGetLastError();
   }
   if constexpr (MX) {
-    // fp32 out tiles: the 256-row tiles' fp32 output does not fit LDS beside
-    // (or inside) their ring, so they give way to 128x128
     if constexpr (sizeof(T) == 2 && EXT && (EPI == EPI_STORE || EPI == EPI_RESID)) {
       if (t == 6 && fits(96)) {
         if (p.k1 % 128 == 0 && p.k2 % 128 == 0)
-          return run<T, 128, 96, 2, 2, 2, EPI, EXT, 16, 10, 256, false, false, false, true>(p, s, false);
-        return run<T, 128, 96, 2, 2, 4, EPI, EXT, 16, 3, 128, false, false, false, true>(p, s, true);
+          return run<T, 128, 96, 2, 2, 2, EPI, EXT, 16, 10, 256, false, false, true>(p, s, false);
+        return run<T, 128, 96, 2, 2, 4, EPI, EXT, 16, 3, 128, false, false, true>(p, s, true);
       }
-      if ((t == 1 || t == 3 || t == 5 || t == 10) && fits(128))
-        return run<T, 128, 128, 2, 2, 4, EPI, EXT, 32, 0, 128, false, false, false, true>(p, s, true);
+      if (t == 1 && fits(128))
+        return run<T, 128, 128, 2, 2, 4, EPI, EXT, 32, 0, 128, false, false, true>(p, s, true);
       if (mixed_tile_ok(t) && fits(64))
-        return run<T, 128, 64, 2, 2, 4, EPI, EXT, 32, 0, 128, false, false, false, true>(p, s, true);
+        return run<T, 128, 64, 2, 2, 4, EPI, EXT, 32, 0, 128, false, false, true>(p, s, true);
     }
     return hipErrorInvalidValue;
   }
   if constexpr (sizeof(T) == 4) {
     if (t == 7) {
-      if (!fits(pl.bn)) return hipErrorInvalidValue;
+      if (!fits(64)) return hipErrorInvalidValue;
       // plain products with long work items (8+ K slices each: the backward's
       // token-contracted products) are load-bound: 4 more waves issue loads
       if constexpr (EPI == EPI_STORE && !EXT) {
@@ -1097,7 +1032,7 @@ hipError_t launch_cmix_value(int dtype, const void* h, const void* wv, int F, co
 // layer 110.3 / 99.8), 8192 x 1024 x 4096 76.9 / 54.1 + 16.0 (230.6 / 223.9), 6000 x
 // 2048 x 8192 bf16 242 / 175 + 17 (458 / 414).
 bool value_combine_fusable(int dtype, int N, int C, int F, int k) {
-  if (dtype == 0 || k < 1 || k > kCombineMaxK || !vs_enabled() || F % 128 || C % 96) return false;
+  if (dtype == 0 || k < 1 || k > kCombineMaxK || F % 128 || C % 96) return false;
   const int cus = num_cus(), tiles = (N + 127) / 128 * (C / 96);
   return tiles <= cus && tiles * 10 >= cus * 9;
 }
@@ -1119,7 +1054,7 @@ hipError_t launch_cmix_value_combine(int dtype, const void* h, const void* wv, i
 }
 
 bool value_sparse_fusable(int dtype, int N, int C, int F, int E, int r, int k, int kx) {
-  if (dtype == 0 || k < 1 || k > kCombineMaxK || !vs_enabled()) return false;
+  if (dtype == 0 || k < 1 || k > kCombineMaxK) return false;
   // one 128-column rank slice per routing rank (kx = 128, the VGPR-staged
   // 128x96 tile's 256-byte K slice), u chunks of 8 columns within one expert
   if (kx != 128 || E * r > kx || r % 8 || E > kSparseMaxE) return false;
@@ -1158,7 +1093,7 @@ hipError_t dispatch_grouped(const GemmParams<T>& p, hipStream_t s) {
     if (pp.cfg < 0) return hipErrorInvalidValue;
     if constexpr (EPI == EPI_KEY)
       if (ring_rows(p.m, p.n, p.k1 / 64, p.grp_n, pp))
-        return run<T, 64, 64, 2, 2, 3, EPI, false, 32, 0, 128, false, false, true>(p, s, false);
+        return run<T, 64, 64, 2, 2, 3, EPI, false, 32, 0, 128, false, true>(p, s, false);
     return pipe_run<T>(p, pp.cfg, EPI == EPI_KEY ? EPI_KEYAD : EPI_STORE, PIPE_GRP, s);
   } else {
     const int cus = num_cus();
@@ -1167,19 +1102,18 @@ hipError_t dispatch_grouped(const GemmParams<T>& p, hipStream_t s) {
       return (long long)((tiles + cus - 1) / cus) * (bm + bn);
     };
     if (p.n % 128 == 0 && cost(128, 128) <= cost(64, 64))
-      return run<T, 128, 128, 2, 2, 3, EPI, false, 32, 0, 128, false, false, true>(p, s, false);
+      return run<T, 128, 128, 2, 2, 3, EPI, false, 32, 0, 128, false, true>(p, s, false);
     if (p.n % 64) return hipErrorInvalidValue;
-    return run<T, 64, 64, 2, 2, 3, EPI, false, 32, 0, 128, false, false, true>(p, s, false);
+    return run<T, 64, 64, 2, 2, 3, EPI, false, 32, 0, 128, false, true>(p, s, false);
   }
 }
 
-// A given plan for the products of the backward (planned by
-// backward_gemm_plan below), or the automatic one.
+// The plan of a product of the backward, as `hint` asks for it.
 TilePlan gemm_nt_plan(int dtype, int m, int n, int k_total, int hint) {
   const int elem = dtype == 0 ? 4 : 2;
   TilePlan pl = plan_tiles(elem, EPI_STORE, m, n, n, k_total);
   // the hints replace only a split plan (products too small to fill the CUs)
-  if (tile_override() != 0 || pl.t != 7) return pl;
+  if (pl.t != 7) return pl;
   const int nkt = k_total / (128 / elem);
   if (hint == GEMM_HINT_NO_SPLIT && n % 64 == 0) {
     // short K (a few slices per tile): unsplit 128x64 tiles, no partials to reduce
@@ -1187,8 +1121,6 @@ TilePlan gemm_nt_plan(int dtype, int m, int n, int k_total, int hint) {
     pl.ks = 1;
   } else if (hint == GEMM_HINT_SPLIT64 && n % 64 == 0) {
     // long K over a small output: 64x64 tiles, K split 8 ways (4 with fewer slices)
-    pl.t = 7;
-    pl.bn = 64;
     pl.ks = 1;
     for (int c : {8, 4, 2})
       if (nkt % c == 0 && nkt / c >= 2) {
@@ -1230,9 +1162,9 @@ hipError_t launch_gemm_grouped_k(int dtype, const void* a, int lda, const void* 
                                     std::max(lda, ldb));
       e = pp.cfg < 0 ? hipErrorInvalidValue : pipe_run<T>(p, pp.cfg, EPI_STORE, PIPE_GK, s);
     } else if (n % 128 == 0) {
-      e = run<T, 128, 128, 2, 2, 3, EPI_STORE, false, 32, 0, 128, false, false, false, false, true>(p, s, false);
+      e = run<T, 128, 128, 2, 2, 3, EPI_STORE, false, 32, 0, 128, false, false, false, true>(p, s, false);
     } else {
-      e = run<T, 64, 64, 2, 2, 3, EPI_STORE, false, 32, 0, 128, false, false, false, false, true>(p, s, false);
+      e = run<T, 64, 64, 2, 2, 3, EPI_STORE, false, 32, 0, 128, false, false, false, true>(p, s, false);
     }
     return mark(e, name, s);
   });

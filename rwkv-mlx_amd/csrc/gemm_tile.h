@@ -203,16 +203,14 @@ RWKV_DEV u32x4 combine_chunk(const GemmParams<T>& p, int gm, int col, u32x4 base
 }
 
 // 16-byte chunk swizzle of an LDS row of RB bytes (RB/16 chunks); the result
-// is always < RB/16.  Rows of 64 B: the 16 (row % 4, chunk) pairs of 16
-// consecutive rows are distinct; rows of 128 B: distinct for rows r and r+8
-// and for rows of either parity; rows of 256 B (a full 64-bank sweep each):
-// distinct over any 16 consecutive rows.  Either way the 16 lanes of one LDS
+// is always < RB/16.  Rows of 128 B: distinct for rows r and r+8 and for rows
+// of either parity; rows of 256 B (a full 64-bank sweep each): distinct over
+// any 16 consecutive rows.  Either way the 16 lanes of one LDS
 // read phase hit distinct banks.
 template <int RB>
 RWKV_DEV int swz(int row) {
-  static_assert(RB == 64 || RB == 128 || RB == 256, "LDS row size");
-  if constexpr (RB == 64) return (row >> 2) & 3;
-  else if constexpr (RB == 128) return (row ^ (row >> 3)) & 7;
+  static_assert(RB == 128 || RB == 256, "LDS row size");
+  if constexpr (RB == 128) return (row ^ (row >> 3)) & 7;
   else return row & 15;
 }
 

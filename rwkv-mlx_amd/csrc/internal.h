@@ -183,14 +183,16 @@ bool value_plan_mixed_ok(int m, int n, int k_total);
 size_t gemm_partial_bytes(int dtype, int m, int n, int n_key, int k_total, bool keyad);
 // out (m x n, row stride ldo) = a1 · b1ᵀ (+ a2 · b2ᵀ when k2 > 0): rows of
 // every operand are K-contiguous; n and the K lengths as for the value GEMM.
-// `hint` picks the tiling for the shapes of the backward (measured):
+// `hint` picks the tiling of an fp32 product that would split K (measured on
+// the backward's shapes); 16-bit products of more than 64 rows have the pipelined
+// tiles' plan whatever it says:
 //   GEMM_HINT_AUTO      the forward's automatic plan;
 //   GEMM_HINT_NO_SPLIT  short K: unsplit 128x64 tiles;
 //   GEMM_HINT_SPLIT64   long K over a small output: 64x64 tiles, K split 8 ways.
 enum { GEMM_HINT_AUTO = 0, GEMM_HINT_NO_SPLIT = 1, GEMM_HINT_SPLIT64 = 2 };
-// With `deferred` not null, a product whose plan splits K leaves its fp32
-// partials part[s][m][n] unreduced and sets *deferred to the split count (1:
-// the product was not split and `out` holds it).
+// With `deferred` not null, a product that splits K on the 64-row tiles (fp32,
+// or 16-bit of at most 64 rows) leaves its fp32 partials part[s][m][n] unreduced
+// and sets *deferred to the split count (1: `out` holds the product).
 hipError_t launch_gemm_nt(int dtype, const void* a1, int lda1, const void* b1, int ldb1, int k1, const void* a2,
                           int lda2, const void* b2, int ldb2, int k2, int m, int n, void* out, int ldo, float* part,
                           const char* name, hipStream_t s, int hint = GEMM_HINT_AUTO, int* deferred = nullptr);
