@@ -777,12 +777,15 @@ unsigned even_tile_rows(int m, int groups, int bm) {
 
 // The tile (and K split) with the least modelled time.  A split adds the
 // reduction's launch, which reads ks partials one after the other, and the fp32
-// partials' way out and back (3.8 TB/s).  A tile never straddles the key / adapter
+// partials' way out and back (3.8 TB/s).  A product of less than 9 us is split
+// only to gain the 2 us of that launch on the host: passes with such products
+// wait for the host (a layer of 81 tokens, 512 x 1792 bf16: 29.0 us unsplit, 30.4
+// in 6 parts).  A tile never straddles the key / adapter
 // column boundary.  groups: row groups or K groups; ld: the operands' row length
 // where it can be long (a tile's rows are addressed with 32 bits).
 PipePlan plan_pipe(int mode, int m, int n, int n_key, int nkt, int groups = 1, long long ld = 0) {
   const int cus = num_cus();
-  PipePlan best{-1, 1, 0.};
+  PipePlan best{-1, 1, 0.}, parts{-1, 1, 0.};
   for (int c = 0; c < kPipeN; ++c) {
     const PipeTile& t = kPipeTiles[c];
     if (n % t.bn || n_key % t.bn || ld * std::max(t.bm, t.bn) * 2 > 0xFFFFFFF0ll) continue;
@@ -799,10 +802,11 @@ PipePlan plan_pipe(int mode, int m, int n, int n_key, int nkt, int groups = 1, l
       // tokens, a third of them skewed, within 0.2% on average)
       if (mode == PIPE_GRP) us = (us + pipe_us(t, even_tile_rows(m, groups, t.bm) * (n / t.bn), nkt, cus)) / 2;
       if (ks > 1) us += 2.75 + 0.05 * ks + (double)ks * m * n * 8.0 / 3.8e6;
-      if (best.cfg < 0 || us < best.us) best = PipePlan{c, ks, us};
+      PipePlan& of = ks > 1 ? parts : best;
+      if (of.cfg < 0 || us < of.us) of = PipePlan{c, ks, us};
     }
   }
-  return best;
+  return parts.cfg >= 0 && parts.us + (best.us < 9.0 ? 2.0 : 0.0) < best.us ? parts : best;
 }
 
 // Whether a row-group key product runs this file's 64x64 ring tile instead: four
