@@ -1,6 +1,6 @@
-// VGPR-staged MFMA GEMM tiles for the layer's two large products (the key
-// projection with relu², model.py:262, and the value projection with the
-// adapter K-extension, model.py:263 / moe.py:139-147).
+// VGPR-staged MFMA GEMM tiles for value products (model.py:263 / moe.py:139-147):
+// the SPARSE layer's with the adapters' rank slices or with the combine in its
+// epilogue, and the fp16 layer's with fp32 adapters.
 //
 // Why a second form: a global_load_lds ring can only have as many K slices
 // in flight as LDS holds free slots, and with two 57 KB slots a CU keeps
@@ -47,7 +47,6 @@ __global__ __launch_bounds__(64 * (WGM * WGN + LW)) void gemm_vs_kernel(GemmPara
   typedef typename M::acc accv;
   constexpr int NMW = WGM * WGN;
   constexpr int NT = 64 * (NMW + LW);
-  static_assert(NT >= kDispThreads, "a dispatch job block needs 256 threads");
   constexpr int VEC = 16 / sizeof(T);
   constexpr int BK = RB / sizeof(T), CPR = RB / 16;
   constexpr int WM = BM / WGM, WN = BN / WGN;
@@ -68,7 +67,6 @@ __global__ __launch_bounds__(64 * (WGM * WGN + LW)) void gemm_vs_kernel(GemmPara
   static_assert(!OUT_IN_RING || 2 * STAGE >= OUT_BYTES, "output tile");
   static_assert(!SP || !OUT_IN_RING, "the rank slices keep the base in the output tile beside the ring");
   static_assert(LDS_BYTES <= 163840, "LDS budget");
-  static_assert(256 + loss_scratch_bytes(NT) <= LDS_BYTES, "loss scratch");
   static_assert(D >= 2 && NPL * (D - 1) < 64, "loads in flight");
   static_assert(M::ACC % 4 == 0, "epilogue writes 4 accumulators at a time");
 
@@ -90,7 +88,6 @@ __global__ __launch_bounds__(64 * (WGM * WGN + LW)) void gemm_vs_kernel(GemmPara
   const int gsize = min(tiles_m - first_m, GROUP_M);
   const int m0 = (first_m + (l % in_group) % gsize) * BM;
   const int n0 = ((l % in_group) / gsize) * BN;
-  const bool adapter = EPI == EPI_KEYAD && n0 >= p.n_key;
 
   const int nk1 = p.k1 / BK;
   const int G = nk1 + (EXT ? p.k2 / BK : 0);  // K slices (EPI_SPARSE: then one per rank)
@@ -128,8 +125,8 @@ __global__ __launch_bounds__(64 * (WGM * WGN + LW)) void gemm_vs_kernel(GemmPara
   const T* src1[NPL];
   const T* src2[EXT ? NPL : 1];
   {
-    const T* A = adapter ? p.a_ad : p.a1;
-    const T* B = adapter ? p.b_ad + (size_t)(n0 - p.n_key) * p.ldb1 : p.b1 + (size_t)n0 * p.ldb1;
+    const T* A = p.a1;
+    const T* B = p.b1 + (size_t)n0 * p.ldb1;
     const int lt = tid - 64 * NMW;
 #pragma unroll
     for (int j = 0; j < NPL; ++j) {
@@ -382,8 +379,6 @@ __global__ __launch_bounds__(64 * (WGM * WGN + LW)) void gemm_vs_kernel(GemmPara
   }
 
   // ---- epilogue ------------------------------------------------------------
-  int ticket = 1;
-  if (p.loss.losses != nullptr && tid == 0) ticket = atomicAdd(p.loss.claim, 1);
   unsigned char* ot = OUT_IN_RING ? lds : lds + 2 * STAGE;
   if (OUT_IN_RING) wait_lds_barrier();  // every MFMA wave is done reading the ring
   if (mma_wave && !SP) {  // (EPI_SPARSE: the tile is already in LDS)
@@ -399,37 +394,10 @@ __global__ __launch_bounds__(64 * (WGM * WGN + LW)) void gemm_vs_kernel(GemmPara
           if constexpr (MX) {  // fp32 out: the accumulators as they are
             *(f32x4*)dst = f32x4{acc[i][j][v0], acc[i][j][v0 + 1], acc[i][j][v0 + 2], acc[i][j][v0 + 3]};
           } else {
-            if constexpr ((EPI == EPI_KEY || EPI == EPI_KEYAD) && std::is_same<T, f16>::value) {
-              if (!adapter) {
-                *(unsigned long long*)dst = relu2_f16x4(acc[i][j][v0], acc[i][j][v0 + 1], acc[i][j][v0 + 2], acc[i][j][v0 + 3]);
-                continue;
-              }
-            }
-            float r[4];
+            union { T e[4]; unsigned long long u; } pk;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) r[q] = rnd<T>(acc[i][j][v0 + q]);
-            if constexpr (EPI == EPI_KEY || EPI == EPI_KEYAD) {
-              if (!adapter) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                  const float z = r[q] > 0.f ? r[q] : 0.f;
-                  r[q] = z * z;  // relu(key(k)) ** 2 (model.py:262)
-                }
-              } else {
-                adapter_scale4(p, min(m0 + row, p.m - 1), n0 - p.n_key + col, r);
-              }
-            }
-            T o[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) o[q] = from_f<T>(r[q]);
-            if constexpr (sizeof(T) == 4) {
-              *(f32x4*)dst = f32x4{to_f(o[0]), to_f(o[1]), to_f(o[2]), to_f(o[3])};
-            } else {
-              union { T e[4]; unsigned long long u; } pk;
-#pragma unroll
-              for (int q = 0; q < 4; ++q) pk.e[q] = o[q];
-              *(unsigned long long*)dst = pk.u;
-            }
+            for (int q = 0; q < 4; ++q) pk.e[q] = from_f<T>(rnd<T>(acc[i][j][v0 + q]));
+            *(unsigned long long*)dst = pk.u;
           }
         }
       }
@@ -469,33 +437,15 @@ __global__ __launch_bounds__(64 * (WGM * WGN + LW)) void gemm_vs_kernel(GemmPara
         }
       }
       if constexpr (EPI == EPI_COMBINE) v = combine_chunk(p, gm, n0 + c, v);
-      T* dstp = adapter ? p.out_ad + (size_t)gm * (p.n - p.n_key) + (n0 - p.n_key) + c
-                        : p.out + (size_t)gm * p.ldo + n0 + c;
-      *(u32x4*)dstp = v;
+      *(u32x4*)(p.out + (size_t)gm * p.ldo + n0 + c) = v;
     }
   }
-  // the router's loss reduction, by the workgroup that took ticket 0
-  if (p.loss.losses != nullptr) {
-    __syncthreads();
-    int* flag = (int*)lds;
-    if (tid == 0) flag[0] = ticket;
-    __syncthreads();
-    const bool mine = flag[0] == 0;
-    __syncthreads();
-    if (mine) {
-      double* sp = (double*)(lds + 256);
-      long long* sc = (long long*)(sp + NT);
-      reduce_losses(p.loss, sp, sc, (double*)(sc + NT));
-    }
-  }
-  // the SPARSE forward's dispatch scatter, block by block (after the tile:
-  // the key product does not read it)
-  dispatch_job_run(p.disp, (int*)lds + 1, (int*)(lds + 256));
 }
 
 template <typename T, int BM, int BN, int WGM, int WGN, int MN, int LW, int RB, int D, int EPI, bool EXT, bool MX>
 hipError_t run_vs(const GemmParams<T>& p, hipStream_t s) {
   constexpr int BK = RB / (int)sizeof(T);
+  if (p.loss.losses || p.disp.nblk > 0) return hipErrorInvalidValue;  // (only key products are given a job)
   if (p.k1 % BK || (EXT && p.k2 % BK) || p.n % BN || p.m < 1) return hipErrorInvalidValue;
   const int tiles = ((p.m + BM - 1) / BM) * (p.n / BN);
   GemmParams<T> q = p;
